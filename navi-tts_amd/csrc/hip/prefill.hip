@@ -15,16 +15,14 @@
 //    N = 1024 fills the 256 CUs. Split-K partials go to a workspace and are summed in a fixed
 //    order by the "finish" kernels, which also apply the epilogue (bias, SiLU, residual):
 //    deterministic results.
-//  * The prefill's layers: five launches each. q|k|v, o, gate|up and down are whole-K row
-//    projections (rows.h) with the input RMSNorm, SwiGLU and the residual add fused in; the q/k
-//    head norms + RoPE and the f16 K/V store run in the q|k|v projection's epilogue (above 64 rows)
-//    or inside the attention (up to 64 rows); then the attention. The
-//    projections read their operands in the MFMA tile layouts (rows.h pk_a / pk_w): a copy of
-//    every layer's weights tiled at create, and the residual stream, the attention output and the
-//    MLP hidden stored tiled by the kernels that write them.
-//  * Causal prefill attention: one block per (row, q head), scores over keys 0..row from the
-//    f16 cache, exactly as the frame's decode attention will later read them.
+//  * The prefill's layers: five launches each. Up to 64 rows q|k|v, o, gate|up and down are whole-K
+//    row projections (rows.h) with the input RMSNorm, SwiGLU and the residual add fused in, and
+//    the attention (one block per row and kv group) applies the q/k head norms + RoPE and stores
+//    the f16 K/V row. Above, gemm.h's projections and attention, which hand every activation on as
+//    f16 pairs in MFMA fragment order. Either way the projections read the weights in the MFMA tile
+//    layout (rows.h pk_w), from a copy of every layer's weights tiled at create.
 #include "dev_common.h"
+#include "gemm.h"
 #include "host_util.h"
 #include "linear.h"
 #include "rows.h"
@@ -210,103 +208,80 @@ __global__ void __launch_bounds__(BT) k_swiglu(const float *part, int S, int M, 
     }
 }
 
-// Causal GQA attention for rows with at most SHORT_KEYS keys (prompts of up to 256 rows; above,
-// k_attn_prefill_long), one block per (row m, kv group g) for its two q heads over keys 0..pos0 + m
-// of the f16 cache (k_prefill_attention, talker.hip:88-117). Wave w takes
-// keys 64w .. 64w + 63; lane 16r + c reads 16-byte chunk c of key 4i + r, so one load instruction
-// covers four whole 256-byte key rows, and every K chunk of the block is issued before the first
-// score (the fused variant stages K and V in LDS; the other issues its V chunks after the scores,
-// so they fly during the softmax and K and V never share the registers): one or two memory
-// latencies per block.
-// Scores are summed over a key's 16 lanes by DPP; thread t owns key t for the softmax.
-// The score and value loops skip the key groups past the row's keys: per group of four keys when
-// every key of the launch falls in wave 0's range (FEW, the fused prompts of up to 64 rows), per
-// wave otherwise (a per-group exit in the unrolled loops of the longer rows measured slower).
+// Causal GQA attention of prompts of up to FUSED_ROWS rows from position 0 (above: gemm.h), one
+// block per (row m, kv group g) for its two q heads over keys 0..m (k_prefill_attention,
+// talker.hip:88-117), with the q/k head norms, RoPE and the f16 K/V store folded in (k_qk_norm_rope,
+// talker.hip:46-82). The block forms, from the raw q|k|v rows of the projection (`raw`, [rows][nq + 2
+// nkv heads] f32), its two q heads and the normed, rotated f16 keys and the f16 values 0..m of kv group
+// g in LDS, one wave per head row (lane l holding dims l and l + 64, the values 0 + x, so a -0 sum is
+// stored as +0), and stores K/V row m into the cache. Then wave w takes keys 64w .. 64w + 63; lane 16r
+// + c holds 16-byte chunk c of key 4i + r. Scores are summed over a key's 16 lanes by DPP; thread t
+// owns key t for the softmax; the score and value loops skip the groups of four keys past the row's.
 constexpr int SHORT_KEYS = 256;
-// FUSED (prompts of up to FUSED_ROWS rows from position 0; FEW): the q/k head norms, RoPE and the
-// f16 K/V store are folded in (k_qk_norm_rope, talker.hip:46-82). The block of row m forms, from
-// the raw q|k|v rows of the projection (`raw`, [rows][nq + 2 nkv heads] f32), its two q heads and
-// the normed, rotated f16 keys and the f16 values 0..m of kv group g in LDS, one wave per head row
-// with the arithmetic of the EPI_QKV epilogue (rows.h: lane l holding dims l and l + 64, the values
-// 0 + x), and it stores K/V row m into the cache; the attention then reads its keys and values from
-// LDS instead of the cache.
 constexpr int FUSED_ROWS = 64;
 struct HeadNorm {
     const float *raw, *qn, *kn, *invf;
     float eps;
 };
-template <bool FEW, bool FUSED = false>
-__global__ void __launch_bounds__(BT) k_attn_prefill_short(const float *q, uint16_t *kc, uint16_t *vc, int nq,
-                                                           int nkv, int pos0, float scale, float *out, int ldo,
-                                                           HeadNorm hn = {}) {
+__global__ void __launch_bounds__(BT) k_attn_prefill_short(uint16_t *kc, uint16_t *vc, int nq, int nkv, float scale, float *out,
+                                                           int ldo, HeadNorm hn) {
     constexpr int NWV = BT / WAVE, KW = SHORT_KEYS / NWV, KI = KW / 4;
     static_assert(SHORT_KEYS == BT, "one key per thread in the softmax");
-    static_assert(FEW == FUSED && (!FUSED || FUSED_ROWS <= KW), "fused (the only FEW case): every key in wave 0's range");
+    static_assert(FUSED_ROWS <= KW, "every key in wave 0's range");
     __shared__ float qs[2][HD], sc[2][SHORT_KEYS], red[2][NWV], opart[NWV][4][2][HD];
-    __shared__ uint16_t ks[FUSED ? FUSED_ROWS : 1][HD], vs[FUSED ? FUSED_ROWS : 1][HD];
+    __shared__ uint16_t ks[FUSED_ROWS][HD], vs[FUSED_ROWS][HD];
     // grid (kv groups, rows): blocks go out in row order from the last row (the most keys) down,
     // every kv group of a row together, so the blocks that wait for a free slot are the shortest;
     // and kv group g's blocks all land on XCD g (block id % 8), whose L2 then holds its keys
-    const int m = static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y), g = blockIdx.x, n = pos0 + m + 1;
+    const int m = static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y), g = blockIdx.x, n = m + 1;
     const int QD = nq * HD, KVD = nkv * HD;
     const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, r = l >> 4;
     u32x4_t kr[KI], vr[KI];
-    if constexpr (FUSED) {
-        // task t: q head 2g + t of row m (t < 2), else key / value row j = t - 2 of kv group g
-        const int W = QD + 2 * KVD;
-        for (int t = wv; t < 2 + n; t += NWV) {
-            const bool isq = t < 2;
-            const int row = isq ? m : t - 2;
-            const float *hp = hn.raw + static_cast<size_t>(row) * W + (isq ? (2 * g + t) * HD : QD + g * HD);
-            const float *vp = hn.raw + static_cast<size_t>(row) * W + QD + KVD + g * HD;
-            const float a0 = 0.f + gld(hp + l), a1 = 0.f + gld(hp + l + HD / 2);
-            float b0 = 0.f, b1 = 0.f;
-            if (!isq) {
-                b0 = 0.f + gld(vp + l);
-                b1 = 0.f + gld(vp + l + HD / 2);
-            }
-            float sn, cs;
-            sincosf(static_cast<float>(row) * gld(hn.invf + l), &sn, &cs);
-            const float *nw = isq ? hn.qn : hn.kn;
-            const float scl = rsqrtf(wave_sum(fmaf(a0, a0, a1 * a1)) / static_cast<float>(HD) + hn.eps);
-            const float x0 = a0 * scl * gld(nw + l), x1 = a1 * scl * gld(nw + l + HD / 2);
-            const float y0 = x0 * cs - x1 * sn;
-            const float y1 = x1 * cs + x0 * sn;
-            if (isq) {
-                qs[t][l] = y0;
-                qs[t][l + HD / 2] = y1;
-            } else {
-                const uint16_t k0 = f2h(y0), k1 = f2h(y1), v0 = f2h(b0), v1 = f2h(b1);
-                ks[row][l] = k0;
-                ks[row][l + HD / 2] = k1;
-                vs[row][l] = v0;
-                vs[row][l + HD / 2] = v1;
-                if (row == m) {
-                    uint16_t *kd = kc + static_cast<size_t>(m) * KVD + g * HD, *vd = vc + static_cast<size_t>(m) * KVD + g * HD;
-                    gst(kd + l, k0);
-                    gst(kd + l + HD / 2, k1);
-                    gst(vd + l, v0);
-                    gst(vd + l + HD / 2, v1);
-                }
-            }
+    // task t: q head 2g + t of row m (t < 2), else key / value row j = t - 2 of kv group g
+    const int W = QD + 2 * KVD;
+    for (int t = wv; t < 2 + n; t += NWV) {
+        const bool isq = t < 2;
+        const int row = isq ? m : t - 2;
+        const float *hp = hn.raw + static_cast<size_t>(row) * W + (isq ? (2 * g + t) * HD : QD + g * HD);
+        const float *vp = hn.raw + static_cast<size_t>(row) * W + QD + KVD + g * HD;
+        const float a0 = 0.f + gld(hp + l), a1 = 0.f + gld(hp + l + HD / 2);
+        float b0 = 0.f, b1 = 0.f;
+        if (!isq) {
+            b0 = 0.f + gld(vp + l);
+            b1 = 0.f + gld(vp + l + HD / 2);
         }
-        __syncthreads();                                  // qs, ks, vs
-#pragma unroll
-        for (int i = 0; i < KI; ++i) {
-            const int j = wv * KW + 4 * i + r;
-            kr[i] = j < n ? *reinterpret_cast<const u32x4_t *>(&ks[j][c * 8]) : u32x4_t{0u, 0u, 0u, 0u};
-            vr[i] = j < n ? *reinterpret_cast<const u32x4_t *>(&vs[j][c * 8]) : u32x4_t{0u, 0u, 0u, 0u};
-        }
-    } else {
-        qs[threadIdx.x >> 7][threadIdx.x & (HD - 1)] = gld(q + static_cast<size_t>(m) * QD + g * 2 * HD + threadIdx.x);
-        const uint16_t *kb = kc + g * HD + c * 8;
-#pragma unroll
-        for (int i = 0; i < KI; ++i) {
-            const int j = wv * KW + 4 * i + r;
-            kr[i] = j < n ? *(const NAVI_GLOBAL u32x4_t *) (kb + static_cast<size_t>(j) * KVD) : u32x4_t{0u, 0u, 0u, 0u};
+        float sn, cs;
+        sincosf(static_cast<float>(row) * gld(hn.invf + l), &sn, &cs);
+        const float *nw = isq ? hn.qn : hn.kn;
+        const float scl = rsqrtf(wave_sum(fmaf(a0, a0, a1 * a1)) / static_cast<float>(HD) + hn.eps);
+        const float x0 = a0 * scl * gld(nw + l), x1 = a1 * scl * gld(nw + l + HD / 2);
+        const float y0 = x0 * cs - x1 * sn;
+        const float y1 = x1 * cs + x0 * sn;
+        if (isq) {
+            qs[t][l] = y0;
+            qs[t][l + HD / 2] = y1;
+        } else {
+            const uint16_t k0 = f2h(y0), k1 = f2h(y1), v0 = f2h(b0), v1 = f2h(b1);
+            ks[row][l] = k0;
+            ks[row][l + HD / 2] = k1;
+            vs[row][l] = v0;
+            vs[row][l + HD / 2] = v1;
+            if (row == m) {
+                uint16_t *kd = kc + static_cast<size_t>(m) * KVD + g * HD, *vd = vc + static_cast<size_t>(m) * KVD + g * HD;
+                gst(kd + l, k0);
+                gst(kd + l + HD / 2, k1);
+                gst(vd + l, v0);
+                gst(vd + l + HD / 2, v1);
+            }
         }
     }
-    __syncthreads();                                      // qs
+    __syncthreads();                                  // qs, ks, vs
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+        const int j = wv * KW + 4 * i + r;
+        kr[i] = j < n ? *reinterpret_cast<const u32x4_t *>(&ks[j][c * 8]) : u32x4_t{0u, 0u, 0u, 0u};
+        vr[i] = j < n ? *reinterpret_cast<const u32x4_t *>(&vs[j][c * 8]) : u32x4_t{0u, 0u, 0u, 0u};
+    }
     {
         float q0[8], q1[8];
 #pragma unroll
@@ -316,7 +291,7 @@ __global__ void __launch_bounds__(BT) k_attn_prefill_short(const float *q, uint1
         }
 #pragma unroll
         for (int i = 0; i < KI; ++i) {
-            if (wv * KW + (FEW ? 4 * i : 0) >= n) break;  // this wave's remaining keys are past the row's
+            if (wv * KW + 4 * i >= n) break;  // this wave's remaining keys are past the row's
             uint4 k4;
             __builtin_memcpy(&k4, &kr[i], 16);
             float a0 = dot8(k4, q0, 0.f), a1 = dot8(k4, q1, 0.f);
@@ -333,17 +308,6 @@ __global__ void __launch_bounds__(BT) k_attn_prefill_short(const float *q, uint1
                 sc[0][j] = a0 * scale;
                 sc[1][j] = a1 * scale;
             }
-        }
-    }
-    if constexpr (!FUSED) {
-        // prompts of 65-256 rows: the V chunks go out after the scores and fly during the softmax,
-        // so K and V are never in registers together (about 100 VGPRs instead of 156: four blocks
-        // per CU instead of three; the sums are unchanged)
-        const uint16_t *vb = vc + g * HD + c * 8;
-#pragma unroll
-        for (int i = 0; i < KI; ++i) {
-            const int j = wv * KW + 4 * i + r;
-            vr[i] = j < n ? *(const NAVI_GLOBAL u32x4_t *) (vb + static_cast<size_t>(j) * KVD) : u32x4_t{0u, 0u, 0u, 0u};
         }
     }
     __syncthreads();
@@ -366,7 +330,7 @@ __global__ void __launch_bounds__(BT) k_attn_prefill_short(const float *q, uint1
         for (int e = 0; e < 8; ++e) o0[e] = o1[e] = 0.f;
 #pragma unroll
         for (int i = 0; i < KI; ++i) {
-            if (wv * KW + (FEW ? 4 * i : 0) >= n) break;  // zero weights (and zero rows) from here on
+            if (wv * KW + 4 * i >= n) break;  // zero weights (and zero rows) from here on
             const int j = wv * KW + 4 * i + r;
             const float p0 = sc[0][j], p1 = sc[1][j];
             half8_t hv;
@@ -393,162 +357,6 @@ __global__ void __launch_bounds__(BT) k_attn_prefill_short(const float *q, uint1
         for (int rr = 0; rr < 4; ++rr) acc += opart[w][rr][hh][d];
     const float sum = red[hh][0] + red[hh][1] + red[hh][2] + red[hh][3];
     gst(out + rows::pk_a(m, (g * 2 + hh) * HD + d, ldo), acc / sum);
-}
-
-// Causal attention of prompts of more than 256 rows on the matrix cores: block (16-row tile qt,
-// q head h) over keys 0..min(T, 16 qt + 16) - 1 of kv group h / (nq / nkv), in chunks of 256 keys
-// with a running softmax. Per chunk: S = Q K^T on v_mfma_f32_16x16x32_f16 with q split into f16
-// hi + lo (f32-level products of the f32 q and the f16 keys; wave w takes the chunk's key tiles w,
-// w + 4, ...), scaled and causally masked into LDS; per row (16 lanes) the chunk's max m_c, the
-// new running max m = max(m_run, m_c), corr = e^(m_run - m), p = e^(s - m) in place, l_run =
-// l_run corr + sum p; the output rows scaled by corr, then O += P V with P split hi + lo against
-// the chunk's V staged transposed in LDS ([dim][key] f16: one 16-byte read per B fragment), wave w
-// taking dims 32w .. 32w + 31. Finally O / l_run to the tile layout of width ldo (rows.h pk_a).
-// Key 0 is in the first chunk of every row, so m_run is finite from the first chunk on.
-constexpr int LONG_CHUNK = 256;
-__global__ void __launch_bounds__(BT) k_attn_prefill_long(const float *q, const uint16_t *kc, const uint16_t *vc, int nq,
-                                                          int nkv, int T, float scale, float *out, int ldo) {
-    constexpr int KT = LONG_CHUNK / 16 / 4;              // key tiles per wave per chunk
-    constexpr int LDS_S = LONG_CHUNK + 4, LDV = LONG_CHUNK + 8;
-    constexpr int VCH = LONG_CHUNK * (HD / 8) / BT;       // 16-byte V chunks per thread per chunk
-    __shared__ float sS[16][LDS_S];
-    __shared__ __align__(16) _Float16 vt[HD][LDV];
-    __shared__ float mrun[16], lrun[16], corr[16];
-    // grid (q heads, row tiles): tiles go out from the last (the most keys) down, every head of a
-    // tile together
-    const int qt = static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y), h = blockIdx.x, g = h / (nq / nkv),
-              r0 = 16 * qt;
-    const int QD = nq * HD, KVD = nkv * HD;
-    const int nk = min(T, r0 + 16);
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, kq = l >> 4;
-    half8_t qh[4], ql[4];
-    {
-        const int row = min(r0 + c, T - 1);
-        const float *qp = q + static_cast<size_t>(row) * QD + h * HD + 8 * kq;
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-            const f32x4_t a0 = ld4(qp + 32 * st), a1 = ld4(qp + 32 * st + 4);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float v = j < 4 ? a0[j] : a1[j - 4];
-                const _Float16 hv = static_cast<_Float16>(v);
-                qh[st][j] = hv;
-                ql[st][j] = static_cast<_Float16>(v - static_cast<float>(hv));
-            }
-        }
-    }
-    if (threadIdx.x < 16) {
-        mrun[threadIdx.x] = -INFINITY;
-        lrun[threadIdx.x] = 0.f;
-    }
-    f32x4_t o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    for (int k0 = 0; k0 < nk; k0 += LONG_CHUNK) {
-        const int nkc = min(LONG_CHUNK, nk - k0), nkt = (nkc + 15) / 16, nks = (nkc + 31) / 32;
-        // the chunk's K fragments and V rows, every load before the first MFMA
-        u32x4_t kf[KT][4];
-#pragma unroll
-        for (int i = 0; i < KT; ++i) {
-            const int kt = w + 4 * i, key = 16 * kt + c;
-#pragma unroll
-            for (int st = 0; st < 4; ++st)
-                kf[i][st] = kt < nkt && key < nkc
-                                ? *(const NAVI_GLOBAL u32x4_t *) (kc + static_cast<size_t>(k0 + key) * KVD + g * HD + 32 * st + 8 * kq)
-                                : u32x4_t{0u, 0u, 0u, 0u};
-        }
-        u32x4_t vch[VCH];
-#pragma unroll
-        for (int i = 0; i < VCH; ++i) {
-            const int e = static_cast<int>(threadIdx.x) + BT * i, key = e / (HD / 8), d8 = e % (HD / 8);
-            vch[i] = key < nkc ? *(const NAVI_GLOBAL u32x4_t *) (vc + static_cast<size_t>(k0 + key) * KVD + g * HD + 8 * d8)
-                               : u32x4_t{0u, 0u, 0u, 0u};
-        }
-        __syncthreads();                                  // the previous chunk's readers of sS, vt are done
-#pragma unroll
-        for (int i = 0; i < KT; ++i) {
-            const int kt = w + 4 * i;
-            if (kt >= nkt) break;
-            f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-                half8_t b;
-                __builtin_memcpy(&b, &kf[i][st], 16);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[st], b, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ql[st], b, acc, 0, 0, 0);
-            }
-            const int key = 16 * kt + c;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = 4 * kq + r;
-                sS[row][key] = key < nkc && k0 + key <= r0 + row ? acc[r] * scale : -INFINITY;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < VCH; ++i) {
-            const int e = static_cast<int>(threadIdx.x) + BT * i, key = e / (HD / 8), d8 = e % (HD / 8);
-            if (key < 32 * nks) {
-                half8_t hv;
-                __builtin_memcpy(&hv, &vch[i], 16);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) vt[8 * d8 + j][key] = hv[j];
-            }
-        }
-        __syncthreads();
-        {
-            // row threadIdx / 16, its 16 lanes take keys lane % 16 + 16 m of the chunk
-            const int row = threadIdx.x >> 4, j0 = threadIdx.x & 15;
-            float mc = -INFINITY;
-            for (int j = j0; j < 32 * nks; j += 16) mc = fmaxf(mc, j < nkt * 16 ? sS[row][j] : -INFINITY);
-            mc = fmaxf(mc, dpp_red<0xB1>(mc));
-            mc = fmaxf(mc, dpp_red<0x4E>(mc));
-            mc = fmaxf(mc, dpp_red<0x141>(mc));
-            mc = fmaxf(mc, dpp_red<0x140>(mc));
-            const float mo = mrun[row], m = fmaxf(mo, mc), cr = expf(mo - m);
-            float sum = 0.f;
-            for (int j = j0; j < 32 * nks; j += 16) {
-                const float e = j < nkt * 16 ? expf(sS[row][j] - m) : 0.f;   // masked: e^-inf = 0
-                sS[row][j] = e;
-                sum += e;
-            }
-            sum += dpp_red<0xB1>(sum);
-            sum += dpp_red<0x4E>(sum);
-            sum += dpp_red<0x141>(sum);
-            sum += dpp_red<0x140>(sum);
-            __syncthreads();                              // every lane of the row has read mrun[row]
-            if (j0 == 0) {
-                mrun[row] = m;
-                lrun[row] = lrun[row] * cr + sum;
-                corr[row] = cr;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[u][r] *= corr[4 * kq + r];
-        for (int t = 0; t < nks; ++t) {
-            half8_t ph, pl;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float v = sS[c][32 * t + 8 * kq + j];
-                const _Float16 hv = static_cast<_Float16>(v);
-                ph[j] = hv;
-                pl[j] = static_cast<_Float16>(v - static_cast<float>(hv));
-            }
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const half8_t b = *reinterpret_cast<const half8_t *>(&vt[32 * w + 16 * u + c][32 * t + 8 * kq]);
-                o[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, b, o[u], 0, 0, 0);
-                o[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, b, o[u], 0, 0, 0);
-            }
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = 4 * kq + r;
-            if (r0 + row < T) gst(out + rows::pk_a(r0 + row, h * HD + 32 * w + 16 * u + c, ldo), o[u][r] / lrun[row]);
-        }
 }
 
 // rows[t] = table[ids[t]] (f16 -> f32), k_gather_rows (talker.hip:20-25).
@@ -651,7 +459,16 @@ struct LayerW {
     const float *ln1, *ln2, *qn, *kn;
     const uint16_t *wq, *wk, *wv, *wo, *wg, *wu, *wd;
     uint16_t *qkv_t, *o_t, *gu_t, *d_t;   // the tiled copies: [q; k; v], o, [gate; up], down
+    float q_scale;                        // gemm.h's scale of the queries (q_scales)
 };
+
+// rot[p] = cos | sin of position p times every inverse frequency.
+__global__ void __launch_bounds__(HD / 2) k_rotation(const float *invf, float *rot) {
+    float sn, cs;
+    sincosf(static_cast<float>(blockIdx.x) * gld(invf + threadIdx.x), &sn, &cs);
+    gst(rot + blockIdx.x * HD + threadIdx.x, cs);
+    gst(rot + blockIdx.x * HD + HD / 2 + threadIdx.x, sn);
+}
 
 // xn = RMSNorm(row m of the tiled residual stream x) * w: k_resid_norm's arithmetic for one row
 // (thread i holds elements 4i .. 4i + 3, the same sum order), reading x in the tile layout.
@@ -697,8 +514,13 @@ struct navi_talker {
     // work buffers
     // x (the residual stream), att and h in the tile layout (rows.h pk_a), the rest row-major
     float *x = nullptr, *xn = nullptr, *q = nullptr, *att = nullptr, *h = nullptr, *part = nullptr, *invf = nullptr;
+    // prompts above FUSED_ROWS rows (gemm.h): the normed residual rows as f16 pairs, their partial sums
+    // of squares, the rotation of every position and the prompt's keys and values as MFMA fragments
+    uint16_t *xs = nullptr, *kf = nullptr, *vf = nullptr;
+    float *ssq = nullptr, *rot = nullptr;
     size_t part_floats = 0;
     uint32_t *flag = nullptr;
+    bool flag_set = false;             // whether a call may have left the flag set
     uint32_t *h_flag = nullptr;        // pinned host copy of flag, read back with the call's last sync
     int32_t *d_ids = nullptr, *d_cids = nullptr, *d_ia = nullptr, *d_ib = nullptr, *d_ta = nullptr, *d_tb = nullptr;
     float *text_rows = nullptr, *fc1_out = nullptr, *proj = nullptr, *codec_rows = nullptr, *spk = nullptr;
@@ -765,6 +587,24 @@ navi_status talker_bind(navi_talker &t, const navi_tensor_ref *tensors, int n_te
     return NAVI_OK;
 }
 
+// The power of two gemm.h's prefill holds a layer's queries in as f16 pairs: 1 unless the norm weights
+// let a query (an RMS-normed, rotated row of 128: at most 16 times the largest weight) leave the f16 range.
+navi_status q_scales(navi_talker &t, char *err, size_t errlen) {
+    std::vector<float> w(static_cast<size_t>(t.L) * HD);
+    for (int l = 0; l < t.L; ++l)
+        NAVI_TRY_HIP(hipMemcpyAsync(w.data() + static_cast<size_t>(l) * HD, t.layers[l].qn, HD * sizeof(float), hipMemcpyDeviceToHost,
+                                    device_state().stream), err, errlen);
+    NAVI_TRY_HIP(hipStreamSynchronize(device_state().stream), err, errlen);
+    for (int l = 0; l < t.L; ++l) {
+        float top = 0.f;
+        for (int i = 0; i < HD; ++i) top = std::max(top, std::fabs(w[static_cast<size_t>(l) * HD + i]));
+        float sc = 1.f;
+        while (std::isfinite(top) && 16.f * top * sc >= 65504.f) sc *= 0.5f;
+        t.layers[l].q_scale = sc;
+    }
+    return NAVI_OK;
+}
+
 // The most partial floats any projection of a prefill (or prompt) of up to M rows needs.
 size_t talker_part_floats(const navi_talker &t) {
     size_t best = 0;
@@ -792,6 +632,7 @@ navi_status flag_result(const navi_talker &t, const char *what, char *err, size_
 navi_status check_flag(navi_talker &t, const char *what, char *err, size_t errlen) {
     NAVI_TRY_HIP(hipMemcpyAsync(t.h_flag, t.flag, 4, hipMemcpyDeviceToHost, device_state().stream), err, errlen);
     NAVI_TRY_HIP(hipStreamSynchronize(device_state().stream), err, errlen);
+    t.flag_set = *t.h_flag != 0;
     return flag_result(t, what, err, errlen);
 }
 
@@ -832,6 +673,7 @@ navi_status navi_talker_create(const navi_model_params *p, const navi_tensor_ref
     t->nothink = p->codec_nothink_id; t->think_bos = p->codec_think_bos_id; t->think_eos = p->codec_think_eos_id;
     auto fail = [&](navi_status s) { delete t; return s; };
     if ((st = talker_bind(*t, tensors, n_tensors, err, errlen)) != NAVI_OK) return fail(st);
+    if ((st = q_scales(*t, err, errlen)) != NAVI_OK) return fail(st);
     const size_t M = t->mmax;
     t->kk.resize(t->L);
     t->vv.resize(t->L);
@@ -847,7 +689,12 @@ navi_status navi_talker_create(const navi_model_params *p, const navi_tensor_ref
     const size_t MT16 = (M + 15) / 16 * 16;     // x, att and h (tile layout) hold whole 16-row tiles
     TALLOC(t->x, MT16 * t->H);
     TALLOC(t->xn, M * t->H);
-    TALLOC(t->q, M * t->QD);
+    TALLOC(t->q, MT16 * t->QD);
+    TALLOC(t->xs, 2 * MT16 * t->H);
+    TALLOC(t->kf, (M + 31) / 32 * 32 * t->KVD);
+    TALLOC(t->vf, (M + 31) / 32 * 32 * t->KVD);
+    TALLOC(t->ssq, gm::SSQ * M);
+    TALLOC(t->rot, M * HD);
     TALLOC(t->att, MT16 * t->QD);
     TALLOC(t->h, MT16 * t->F);
     const size_t per_layer = static_cast<size_t>(t->QD + 2 * t->KVD) * t->H + static_cast<size_t>(t->H) * t->QD +
@@ -900,8 +747,12 @@ navi_status navi_talker_create(const navi_model_params *p, const navi_tensor_ref
             p += static_cast<size_t>(t->H) * t->F;
         }
     }
-    if (hipMemcpyAsync(t->invf, invf, sizeof invf, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipEventCreate(&t->ev0) != hipSuccess || hipEventCreate(&t->ev1) != hipSuccess ||
+    if (hipMemcpyAsync(t->invf, invf, sizeof invf, hipMemcpyHostToDevice, s) != hipSuccess) {
+        set_err(err, errlen, "talker: HIP setup failed");
+        return fail(NAVI_ERR_HIP);
+    }
+    hipLaunchKernelGGL(k_rotation, dim3(static_cast<unsigned>(M)), dim3(HD / 2), 0, s, t->invf, t->rot);
+    if (hipEventCreate(&t->ev0) != hipSuccess || hipEventCreate(&t->ev1) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void **>(&t->h_flag), 64, hipHostMallocDefault) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
         set_err(err, errlen, "talker: HIP setup failed");
@@ -977,6 +828,7 @@ navi_status navi_talker_build_prompt(navi_talker *t, const int32_t *ids, int32_t
 
     hipStream_t s = device_state().stream;
     NAVI_TRY_HIP(hipMemsetAsync(t->flag, 0, 4, s), err, errlen);
+    t->flag_set = true;
     NAVI_TRY_HIP(hipMemcpyAsync(t->d_ids, tids.data(), tids.size() * 4, hipMemcpyHostToDevice, s), err, errlen);
     NAVI_TRY_HIP(hipMemcpyAsync(t->d_cids, cids.data(), cids.size() * 4, hipMemcpyHostToDevice, s), err, errlen);
     NAVI_TRY_HIP(hipMemcpyAsync(t->spk, speaker, t->H * 4, hipMemcpyHostToDevice, s), err, errlen);
@@ -1016,34 +868,75 @@ navi_status navi_talker_build_prompt(navi_talker *t, const int32_t *ids, int32_t
 
 namespace {
 
-// The prefill's kernels for T rows already in t.x (tile layout): five launches per layer (q|k|v
-// with the RMSNorm fused, and above 64 rows the q/k norms + RoPE + K/V store in its epilogue ->
-// attention (up to 64 rows with the norms, RoPE and K/V store) -> o (+ residual) -> gate|up with
-// the RMSNorm and SwiGLU fused -> down (+ residual); every projection one whole-K MFMA kernel on
-// the tiled operands, rows.h), then the last row's final RMSNorm (the post-norm hidden the frame
-// takes) and the codec head. false: a projection shape the tiled kernels do not take (nothing
-// after it was launched).
+// The prefill's kernels for T rows already in t.x (tile layout): five launches per layer, then the
+// last row's final RMSNorm (the post-norm hidden the frame takes) and the codec head. Up to FUSED_ROWS
+// rows: q|k|v with the RMSNorm fused -> attention with the q/k norms, RoPE and the K/V store -> o (+
+// residual) -> gate|up with the RMSNorm and SwiGLU fused -> down (+ residual), every projection one
+// whole-K MFMA kernel on the tiled operands (rows.h). Above: gemm.h's kernels, every activation
+// handed on as f16 pairs in fragment order (t.xs and t.ssq from k_split_rows). false: a projection
+// shape the tiled kernels do not take (nothing after it was launched).
 bool prefill_layers(navi_talker &t, int T, hipStream_t s) {
     const int H = t.H, QKVW = t.QD + 2 * t.KVD;
     const float scale = 1.f / std::sqrt(static_cast<float>(HD));
     for (int l = 0; l < t.L; ++l) {
         const LayerW &w = t.layers[l];
-        if (T <= FUSED_ROWS) {         // the q/k norms, RoPE and K/V store inside the attention
-            if (!rows::launch_rows_pk(rows::EPI_PLAIN, true, t.x, T, H, w.ln1, t.eps, w.qkv_t, QKVW, t.part, QKVW, t.flag, s))
-                return false;
-            hipLaunchKernelGGL((k_attn_prefill_short<true, true>), dim3(t.NKV, T), dim3(BT), 0, s, nullptr, t.kk[l],
-                               t.vv[l], t.NQ, t.NKV, 0, scale, t.att, t.QD, HeadNorm{t.part, w.qn, w.kn, t.invf, t.eps});
-        } else {                       // ... or in the q|k|v projection's epilogue
-            const rows::HeadOut ho{w.qn, w.kn, t.invf, t.q, t.kk[l], t.vv[l], t.NQ, t.NKV, 0};
-            if (!rows::launch_rows_pk(rows::EPI_QKV, true, t.x, T, H, w.ln1, t.eps, w.qkv_t, QKVW, nullptr, 0, t.flag, s, ho))
-                return false;
-            if (T <= SHORT_KEYS)
-                hipLaunchKernelGGL(k_attn_prefill_short<false>, dim3(t.NKV, T), dim3(BT), 0, s, t.q, t.kk[l], t.vv[l], t.NQ,
-                                   t.NKV, 0, scale, t.att, t.QD, HeadNorm{});
-            else
-                hipLaunchKernelGGL(k_attn_prefill_long, dim3(t.NQ, (T + 15) / 16), dim3(BT), 0, s, t.q, t.kk[l], t.vv[l],
-                                   t.NQ, t.NKV, T, scale, t.att, t.QD);
+        if (T > FUSED_ROWS) {
+            auto half = [](float *p) { return reinterpret_cast<uint16_t *>(p); };
+            gm::GemmArgs a{};
+            a.flag = t.flag;
+            a.M = T;
+            a.eps = t.eps;
+            a.ssq_in = a.ssq_out = t.ssq;
+            a.ldq = t.mmax;
+            gm::GemmArgs b = a;
+            b.x = t.xs;
+            b.w = w.qkv_t;
+            b.K = H;
+            b.N = QKVW;
+            b.qn = w.qn;
+            b.kn = w.kn;
+            b.cs = t.rot;
+            b.q = half(t.q);
+            b.kc = t.kk[l];
+            b.vc = t.vv[l];
+            b.kf = t.kf;
+            b.vf = t.vf;
+            b.q_scale = w.q_scale;
+            b.nq = t.NQ;
+            b.nkv = t.NKV;
+            gm::launch_qkv(b, s);
+            hipLaunchKernelGGL(gm::k_attn_prompt, dim3(t.NKV, (T + 15) / 16), dim3(4 * WAVE), 0, s,
+                               gm::AttnArgs{half(t.q), t.kf, t.vf, half(t.att), t.flag, T, t.NQ, scale / w.q_scale});
+            b = a;
+            b.x = half(t.att);
+            b.w = w.o_t;
+            b.K = t.QD;
+            b.N = H;
+            b.res = t.x;
+            b.ln = w.ln2;
+            b.y = t.xs;
+            gm::launch_resid<64>(b, s);
+            b = a;
+            b.x = t.xs;
+            b.w = w.gu_t;
+            b.K = H;
+            b.N = t.F;
+            b.y = half(t.h);
+            gm::launch_gate_up(b, s);
+            b = a;
+            b.x = half(t.h);
+            b.w = w.d_t;
+            b.K = t.F;
+            b.N = H;
+            b.res = t.x;
+            b.ln = l + 1 < t.L ? t.layers[l + 1].ln1 : nullptr;
+            b.y = t.xs;
+            gm::launch_resid<96>(b, s);
+            continue;
         }
+        if (!rows::launch_rows_pk(rows::EPI_PLAIN, true, t.x, T, H, w.ln1, t.eps, w.qkv_t, QKVW, t.part, QKVW, t.flag, s)) return false;
+        hipLaunchKernelGGL(k_attn_prefill_short, dim3(t.NKV, T), dim3(BT), 0, s, t.kk[l], t.vv[l], t.NQ, t.NKV, scale, t.att, t.QD,
+                           HeadNorm{t.part, w.qn, w.kn, t.invf, t.eps});
         if (!rows::launch_rows_pk(rows::EPI_RESID, false, t.att, T, t.QD, nullptr, 0.f, w.o_t, H, t.x, 0, t.flag, s) ||
             !rows::launch_rows_pk(rows::EPI_SWIGLU, true, t.x, T, H, w.ln2, t.eps, w.gu_t, t.F, t.h, 0, t.flag, s) ||
             !rows::launch_rows_pk(rows::EPI_RESID, false, t.h, T, t.F, nullptr, 0.f, w.d_t, H, t.x, 0, t.flag, s))
@@ -1073,7 +966,14 @@ navi_status navi_talker_prefill(navi_talker *t, const float *d_rows, int32_t n_r
     const int T = n_rows, H = t->H;
     hipStream_t s = device_state().stream;
     NAVI_TRY_HIP(hipEventRecord(t->ev0, s), err, errlen);
-    rows::tile_rows(d_rows, T, H, t->x, s, t->flag);       // also clears the f16-range flag
+    // the rows into the layers' layout; the f16-range flag is clear when the layers start
+    if (T > FUSED_ROWS) {
+        if (t->flag_set) NAVI_TRY_HIP(hipMemsetAsync(t->flag, 0, 4, s), err, errlen);
+        hipLaunchKernelGGL(gm::k_split_rows, dim3(T), dim3(256), 0, s, d_rows, t->layers[0].ln1, t->x, t->xs, t->ssq, t->mmax, t->flag);
+    } else {
+        rows::tile_rows(d_rows, T, H, t->x, s, t->flag);
+    }
+    t->flag_set = true;
     // The layers and the head: a launch sequence that depends only on T (every buffer is the
     // handle's), so it can be captured once per row count as a HIP graph and replayed
     // (navi_talker_set_graphs; off by default, measured no faster than host launches).
@@ -1108,6 +1008,7 @@ navi_status navi_talker_prefill(navi_talker *t, const float *d_rows, int32_t n_r
     float ms = 0.f;
     NAVI_TRY_HIP(hipEventElapsedTime(&ms, t->ev0, t->ev1), err, errlen);
     t->last_ms = ms;
+    t->flag_set = *t->h_flag != 0;
     const navi_status st = flag_result(*t, "prefill", err, errlen);
     if (st != NAVI_OK) return st;
     t->n_used = T;

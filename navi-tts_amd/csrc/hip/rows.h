@@ -19,18 +19,7 @@ namespace rows {
 // (sums taken in a fixed order, the same in every block) multiplies the results. Epilogues:
 // plain store, SiLU(gate) * up, or an add into the residual stream. No split-K partials and no
 // finish kernels: at these sizes the launch count is what bounds a layer.
-enum { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_RESID = 2, EPI_QKV = 3 };
-
-// EPI_QKV: the q|k|v projection of a prompt with the per-head work of the attention's input in its
-// epilogue: q and k heads RMSNorm'd (qn / kn) and rotated (rotate-half RoPE at position pos0 + m),
-// q kept f32 in q [M][nq 128], k and v rounded to f16 into the cache rows kc / vc [pos][nkv 128].
-// A block owns one 128-wide head of 16 rows (talker.hip:46-82's k_qk_norm_rope).
-struct HeadOut {
-    const float *qn, *kn, *invf;
-    float *q;
-    uint16_t *kc, *vc;
-    int nq, nkv, pos0;
-};
+enum { EPI_PLAIN = 0, EPI_SWIGLU = 1, EPI_RESID = 2 };
 
 struct RowArgs {
     const float *a;                   // A [M][lda] f32
@@ -42,7 +31,6 @@ struct RowArgs {
     float eps;
     const float *rs;                  // RESID: per-column scale of the added product (a layer scale), or null
     int ypk;                          // packed kernels: y's width for a SWIGLU / RESID output in the tile layout
-    HeadOut ho;                       // EPI_QKV
     int ars = 1, aoff = 0;            // packed kernels: row m of the product reads row m * ars + aoff of A
 };
 
@@ -79,9 +67,7 @@ template <int MT, int EPI, bool NORM, int NWV, int KS, int CG = 1, bool PK = fal
 __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
     constexpr int NT = EPI == EPI_SWIGLU ? 2 : 1, K = 32 * KS * NWV;
     static_assert(CG * MT <= NWV, "one finishing wave per output tile");
-    static_assert(EPI != EPI_QKV || (MT == 1 && CG == 8 && NWV >= 8), "EPI_QKV: one 128-wide head of 16 rows per block");
     __shared__ f32x4_t red[NWV][NT][CG][MT][WAVE];
-    __shared__ float hs[EPI == EPI_QKV ? 16 : 1][EPI == EPI_QKV ? 128 : 1];
     __shared__ float ssq[NWV][MT][WAVE];
     __shared__ float rscale[MT * 16];
     const int w = static_cast<int>(threadIdx.x) / WAVE, l = static_cast<int>(threadIdx.x) & (WAVE - 1);
@@ -231,10 +217,6 @@ __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
             const int mr = 16 * i + 4 * kq + r, m = m0 + mr;
             if (m >= a.M) continue;
             const float sc = NORM ? rscale[mr] : 1.f;
-            if constexpr (EPI == EPI_QKV) {
-                hs[mr][16 * g + c] = v[0][r] * sc;
-                continue;
-            }
             float *dst = a.y + (PK && EPI != EPI_PLAIN ? pk_a(m, nb, a.ypk) : static_cast<size_t>(m) * a.ldy + nb);
             if constexpr (EPI == EPI_PLAIN) {
                 *dst = v[0][r] * sc;
@@ -243,40 +225,6 @@ __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
                 *dst = g / (1.f + expf(-g)) * u;
             } else {
                 *dst = a.rs ? v[0][r] * rsc + old[r] : old[r] + v[0][r];
-            }
-        }
-    }
-    if constexpr (EPI == EPI_QKV) {
-        // one wave per (row, head): lane l holds dims l and l + 64 (the values 0 + x, so a -0 sum
-        // is stored as +0), the same arithmetic as a separate norm/RoPE pass over the stored rows
-        __syncthreads();
-        const HeadOut &o = a.ho;
-        const int hh = blockIdx.x, QD = o.nq * 128, KVD = o.nkv * 128;
-        for (int r2 = 2 * w; r2 < 2 * w + 2 && w < 8; ++r2) {
-            const int m = m0 + r2, pos = o.pos0 + m;
-            if (m >= a.M) break;
-            const float a0 = 0.f + hs[r2][l], a1 = 0.f + hs[r2][l + 64];
-            if (hh >= o.nq + o.nkv) {
-                uint16_t *vd = o.vc + static_cast<size_t>(pos) * KVD + (hh - o.nq - o.nkv) * 128;
-                gst(vd + l, f2h(a0));
-                gst(vd + l + 64, f2h(a1));
-                continue;
-            }
-            float sn, cs;
-            sincosf(static_cast<float>(pos) * gld(o.invf + l), &sn, &cs);
-            const float *nw = hh < o.nq ? o.qn : o.kn;
-            const float sc = rsqrtf(wave_sum(fmaf(a0, a0, a1 * a1)) / 128.f + a.eps);
-            const float x0 = a0 * sc * gld(nw + l), x1 = a1 * sc * gld(nw + l + 64);
-            const float y0 = x0 * cs - x1 * sn;
-            const float y1 = x1 * cs + x0 * sn;
-            if (hh < o.nq) {
-                float *qd = o.q + static_cast<size_t>(m) * QD + hh * 128;
-                gst(qd + l, y0);
-                gst(qd + l + 64, y1);
-            } else {
-                uint16_t *kd = o.kc + static_cast<size_t>(pos) * KVD + (hh - o.nq) * 128;
-                gst(kd + l, f2h(y0));
-                gst(kd + l + 64, f2h(y1));
             }
         }
     }
@@ -372,7 +320,7 @@ void launch_pk(int M, int N, const RowArgs &ra, hipStream_t s) {
     hipLaunchKernelGGL((k_rows<MT, EPI, NORM, NWV, KS, CG, true>), grid, dim3(NWV * WAVE), 0, s, ra);
 }
 
-// The prompt prefill's projections on the tile layouts (talker shapes: K 1024 into q|k|v and gate|up,
+// The projections of the multi-stream decode and of short prompts on the tile layouts (talker shapes: K 1024 into q|k|v and gate|up,
 // 2048 into o, 3072 into down). A: [M][K] tiled; W: one [N][K] tiled matrix (q|k|v and gate|up
 // stacked); y: PLAIN row-major [M][ldy], SWIGLU ([M][F]) and RESID ([M][N]) tiled. Tile shapes from a
 // sweep at 10 and 130 rows (weights streamed from HBM): above 64 rows 16-row tiles with 8 (q|k|v),
@@ -380,20 +328,13 @@ void launch_pk(int M, int N, const RowArgs &ra, hipStream_t s) {
 // shape keeps the row-major kernels' split of K over the waves, so the outputs are theirs bit for
 // bit (gate|up over 16 waves x 2 steps measured 0.7 us faster at 130 rows, with other bits).
 // false: a shape these kernels do not take.
-// EPI_QKV (above 64 rows, talker heads of 128 with ho): the q|k|v projection with the head norms,
-// RoPE and the K/V store in its epilogue; y is not written.
 bool launch_rows_pk(int epi, bool norm, const float *A, int M, int K, const float *ln, float eps, const uint16_t *w, int N,
-                    float *y, int ldy, uint32_t *flag, hipStream_t s, const HeadOut &ho = {}, int ars = 1, int aoff = 0) {
+                    float *y, int ldy, uint32_t *flag, hipStream_t s, int ars = 1, int aoff = 0) {
     const int F = epi == EPI_SWIGLU ? N : 0;
     const RowArgs ra{A, ln, w, nullptr, nullptr, y, flag, 0, M, K, epi == EPI_SWIGLU ? 2 * N : N, epi == EPI_SWIGLU ? 2 * N : N,
-                     F, ldy, eps, nullptr, N, ho, ars, aoff};
+                     F, ldy, eps, nullptr, N, ars, aoff};
     if (M < 1 || N % 128 != 0 || (epi == EPI_SWIGLU && !norm) || ars < 1 || aoff < 0) return false;
     const bool wide = M > 64;
-    if (epi == EPI_QKV) {
-        if (!wide || !norm || K != 1024 || N != 128 * (ho.nq + 2 * ho.nkv)) return false;
-        launch_pk<1, EPI_QKV, true, 8, 4, 8>(M, N, ra, s);
-        return true;
-    }
     // up to 64 rows: 16-row tiles up to 32 rows (faster than 32-row tiles there), 32-row tiles for
     // q|k|v and a whole-M tile for gate|up above (the sweep's best at 64 rows)
     if (epi == EPI_PLAIN && norm && K == 1024) {

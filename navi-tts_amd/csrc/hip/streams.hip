@@ -714,8 +714,8 @@ navi_status run_group(navi_streams *h, StreamWork &g, int i0, int n, int zsplits
             if (!ok) return unsupported(err, errlen);
         }
         // the cp norm and lm_head[pos - 1] on the last row of each stream (row m T + T - 1 of x)
-        if (!launch_rows_pk(EPI_PLAIN, true, g.x, n, H, h->cp_norm, ec, h->lm_head_t[pos - 1], h->VC, g.lg, h->VC, h->flag, s, {},
-                            T, T - 1))
+        if (!launch_rows_pk(EPI_PLAIN, true, g.x, n, H, h->cp_norm, ec, h->lm_head_t[pos - 1], h->VC, g.lg, h->VC, h->flag, s, T,
+                            T - 1))
             return unsupported(err, errlen);
         if (h->taps_on)
             NAVI_TRY_HIP(hipMemcpy2DAsync(h->tap_cp() + (static_cast<size_t>(i0) * CPH + (pos - 1)) * h->VC,
