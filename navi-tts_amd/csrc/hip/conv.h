@@ -56,9 +56,56 @@ struct ConvArgs {
 
 __device__ __forceinline__ float silu(float g) { return g / (1.f + expf(-g)); }
 
+// sin^2(u). Its period is pi and it is even, so no quadrant has to be told apart: r = u - n pi, |r| <= pi /
+// 2 (pi as two floats; the first product is exact and so is its difference from u), then a polynomial
+// in z = r^2, z + z^2 P(z) with P fitted to (sin^2(sqrt z) - z) / z^2 (least squares on Chebyshev nodes,
+// reweighted towards the smallest maximum: 2e-10 over |r| <= 1.64). 13 instructions where sinf(u)^2 takes
+// about three times as many and a branch to its reduction for large arguments at every use: the
+// epilogues' sines took longer than their MFMAs (last decoder block's residual unit at 240 frames 394
+// -> 289 us, a 240-frame block 5.50 -> 4.84 ms, 52 streamed frames 3.69 -> 3.45). Root mean square
+// error 3.4e-8 for |u| up to 2^20 (a correctly rounded sinf squared: 2.7e-8); the PCM's distance from 64
+// bits stays 1.2e-6. Larger arguments, which no activation inside the f16 range gives with a sane
+// alpha, reduce in double.
+constexpr float SIN2_MAX = 1048576.f;
+__device__ __forceinline__ float sin2_poly(float r) {
+    const float z = r * r;
+    float p = fmaf(7.925196854330352e-8f, z, -4.2174178815912455e-6f);
+    p = fmaf(p, z, 1.40975636895746e-4f);
+    p = fmaf(p, z, -3.174476558342576e-3f);
+    p = fmaf(p, z, 4.444437846541405e-2f);
+    p = fmaf(p, z, -3.333333134651184e-1f);
+    return fmaf(z * z, p, z);
+}
+__device__ __forceinline__ float sin2_reduce(float u) {
+    const float n = rintf(u * 0.318309873f);
+    return fmaf(-n, -8.74227766e-8f, fmaf(-n, 3.14159274f, u));
+}
+__device__ __forceinline__ float sin2_reduce_wide(float u) {
+    const double m = rint(static_cast<double>(u) * 0.3183098861837907);
+    return static_cast<float>(fma(-m, 1.2246467991473532e-16, fma(-m, 3.141592653589793, static_cast<double>(u))));
+}
+
+// v + zb sin^2(za v) for N values of one channel: one branch for all of them, their chains interleaved.
+template <int N>
+__device__ __forceinline__ void snake_n(const float (&v)[N], float za, float zb, float (&out)[N]) {
+    float big = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) big = fmaxf(big, fabsf(v[i] * za));
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = sin2_reduce(v[i] * za);
+    if (__builtin_expect(big > SIN2_MAX, 0)) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if (fabsf(v[i] * za) > SIN2_MAX) out[i] = sin2_reduce_wide(v[i] * za);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = fmaf(sin2_poly(out[i]), zb, v[i]);
+}
 __device__ __forceinline__ float snake(float v, float za, float zb) {
-    const float sn = sinf(v * za);
-    return v + sn * sn * zb;
+    const float a[1] = {v};
+    float o[1];
+    snake_n(a, za, zb, o);
+    return o[0];
 }
 
 // The per-output-channel operands of the epilogue, loaded once per thread (a thread's outputs
@@ -82,7 +129,7 @@ __device__ __forceinline__ bool epi_has_res(int epi) { return epi == EPI_RESIDUA
 // residual at o, loaded by the caller before any of its stores (the residual stream is usually
 // y itself, so a load after a store could not be hoisted and every output would wait a memory
 // round trip).
-__device__ __forceinline__ void conv_store(const ConvArgs &a, int epi, size_t o, const EpiCol &c, float v, float res) {
+__device__ __forceinline__ float conv_value(const ConvArgs &a, int epi, const EpiCol &c, float v, float res) {
     if (a.bias) v += c.bias;
     if (epi == EPI_GELU) v = 0.5f * v * (1.f + erff(v * 0.70710678118654752f));
     else if (epi == EPI_RESIDUAL) v += res;
@@ -91,6 +138,10 @@ __device__ __forceinline__ void conv_store(const ConvArgs &a, int epi, size_t o,
     else if (epi == EPI_RELU) v = fmaxf(v, 0.f);
     else if (epi == EPI_SIGMOID) v = 1.f / (1.f + expf(-v));
     else if (epi == EPI_RELU_TANH) v = tanhf(fmaxf(v, 0.f));
+    return v;
+}
+__device__ __forceinline__ void conv_store(const ConvArgs &a, int epi, size_t o, const EpiCol &c, float v, float res) {
+    v = conv_value(a, epi, c, v, res);
     if (a.y) gst(a.y + o, v);
     if (a.z) gst(a.z + o, snake(v, c.za, c.zb));
 }
@@ -514,12 +565,20 @@ __global__ void __launch_bounds__(BT) k_conv_wide(ConvArgs a) {
                             ? gld(a.res + (static_cast<size_t>(t) * a.phases + phase) * a.ldy + co) : 0.f;
         }
 #pragma unroll
-    for (int c = 0; c < NCT; ++c)
+    for (int c = 0; c < NCT; ++c) {
+        const int co = n0 + wc + 32 * c + (l & 31);
+        float v[16], z[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = conv_value(a, EPI, cc[c], acc[c][r], res[c][r]);
+        if (a.z) snake_n(v, cc[c].za, cc[c].zb, z);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int t = t0 + wr + 8 * (r / 4) + 4 * (l >> 5) + (r & 3), co = n0 + wc + 32 * c + (l & 31);
-            if (t < a.T) conv_store(a, EPI, (static_cast<size_t>(t) * a.phases + phase) * a.ldy + co, cc[c], acc[c][r], res[c][r]);
+            const int t = t0 + wr + 8 * (r / 4) + 4 * (l >> 5) + (r & 3);
+            const size_t o = (static_cast<size_t>(t) * a.phases + phase) * a.ldy + co;
+            if (t < a.T && a.y) gst(a.y + o, v[r]);
+            if (t < a.T && a.z) gst(a.z + o, z[r]);
         }
+    }
     if (a.hnext) carry_rows(a.hist, a.x, a.ldx, a.T, H, a.Cin, a.hnext);
 }
 
@@ -803,17 +862,21 @@ __global__ void __launch_bounds__(BT) k_unit(UnitArgs u) {
         zbm[c] = gld(u.zb_mid + co);
     }
     __syncthreads();                                        // every wave is done with the k7 staging
+    if (mma)
 #pragma unroll
-    for (int c = 0; c < NCT; ++c)
+        for (int c = 0; c < NCT; ++c) {
+            float v[16], z[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            if (!mma) break;
-            const int row = wr + 8 * (r / 4) + 4 * (l >> 5) + (r & 3), co = wc + 32 * c + (l & 31);
-            const float m = snake(acc[c][r] + b7c[c], zam[c], zbm[c]);
-            if (t0 + row < u.T) bad |= !(fabsf(m) < 65504.f);
-            const _Float16 h = static_cast<_Float16>(m);
-            mhi[row * LDM + co] = h;
-            mlo[row * LDM + co] = static_cast<_Float16>(m - static_cast<float>(h));
+            for (int r = 0; r < 16; ++r) v[r] = acc[c][r] + b7c[c];
+            snake_n(v, zam[c], zbm[c], z);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = wr + 8 * (r / 4) + 4 * (l >> 5) + (r & 3), co = wc + 32 * c + (l & 31);
+                if (t0 + row < u.T) bad |= !(fabsf(z[r]) < 65504.f);
+                const _Float16 h = static_cast<_Float16>(z[r]);
+                mhi[row * LDM + co] = h;
+                mlo[row * LDM + co] = static_cast<_Float16>(z[r] - static_cast<float>(h));
+            }
         }
     if (bad) gst(u.flag, 1u);
     // ---- k1: 32-channel weight pieces, 16-channel steps in channel order, hi then lo ----
@@ -864,16 +927,21 @@ __global__ void __launch_bounds__(BT) k_unit(UnitArgs u) {
         }
     }
 #pragma unroll
-    for (int c = 0; c < NCT; ++c)
+    for (int c = 0; c < NCT; ++c) {
+        const int co = wc + 32 * c + (l & 31);
+        float v[16], z[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = (acc1[c][r] + b1c[c]) + rs[c][r];
+        snake_n(v, zac[c], zbc[c], z);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int t = t0 + wr + 8 * (r / 4) + 4 * (l >> 5) + (r & 3), co = wc + 32 * c + (l & 31);
+            const int t = t0 + wr + 8 * (r / 4) + 4 * (l >> 5) + (r & 3);
             if (t >= u.T) continue;
-            const float v = (acc1[c][r] + b1c[c]) + rs[c][r];
             const size_t o = static_cast<size_t>(t) * C + co;
-            if (u.y) gst(u.y + o, v);
-            gst(u.z + o, snake(v, zac[c], zbc[c]));
+            if (u.y) gst(u.y + o, v[r]);
+            gst(u.z + o, z[r]);
         }
+    }
     if (u.hnext) carry_rows(u.hist, u.x, C, u.T, H, C, u.hnext);
 }
 
