@@ -63,8 +63,11 @@ typedef _Float16 rhalf8 __attribute__((ext_vector_type(8)));
 // N / (16 CG) times per launch instead of N / 16. A column's sums are the same at any CG.
 // PK: A, W and a SWIGLU / RESID y in the tile layouts above (W one [N][K] matrix in w0, y of width
 // a.ypk); the same products in the same order, so the same bits as the row-major kernel.
-template <int MT, int EPI, bool NORM, int NWV, int KS, int CG = 1, bool PK = false>
+// CS > 1 (one column group): CS blocks share the 16 columns of a weight tile, each storing 16 / CS of them
+// and reading only those rows of the tile (the others' operands are zeros): the same sums, over more CUs.
+template <int MT, int EPI, bool NORM, int NWV, int KS, int CG = 1, bool PK = false, int CS = 1>
 __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
+    static_assert(CS == 1 || (CG == 1 && PK), "a split weight tile");
     constexpr int NT = EPI == EPI_SWIGLU ? 2 : 1, K = 32 * KS * NWV;
     static_assert(CG * MT <= NWV, "one finishing wave per output tile");
     __shared__ f32x4_t red[NWV][NT][CG][MT][WAVE];
@@ -72,7 +75,9 @@ __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
     __shared__ float rscale[MT * 16];
     const int w = static_cast<int>(threadIdx.x) / WAVE, l = static_cast<int>(threadIdx.x) & (WAVE - 1);
     const int c = l & 15, kq = l >> 4, m0 = blockIdx.y * (MT * 16);
-    const int nb0 = blockIdx.x * (16 * CG) + c;        // column of group 0; group g: nb0 + 16 g
+    const int cb = static_cast<int>(blockIdx.x) / CS;  // column block
+    const int nb0 = cb * (16 * CG) + c;                // column of group 0; group g: nb0 + 16 g
+    const bool mycol = CS == 1 || c / (16 / CS) == static_cast<int>(blockIdx.x) % CS;
     auto wrow = [&](int n) {
         return n < a.n1 ? a.w0 + static_cast<size_t>(n) * K
              : n < a.n2 ? a.w1 + static_cast<size_t>(n - a.n1) * K : a.w2 + static_cast<size_t>(n - a.n2) * K;
@@ -95,8 +100,10 @@ __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
 #pragma unroll
                 for (int g = 0; g < CG; ++g) {
                     if constexpr (PK) {
-                        const int n = (t ? a.F : 0) + blockIdx.x * (16 * CG) + 16 * g;
-                        bv[t][g][st] = *(const NAVI_GLOBAL u32x4_t *) (a.w0 + (static_cast<size_t>(n >> 4) * (K / 32) + w * KS + st) * 512 + l * 8);
+                        const int n = (t ? a.F : 0) + cb * (16 * CG) + 16 * g;
+                        u32x4_t b = {0u, 0u, 0u, 0u};
+                        if (mycol) b = *(const NAVI_GLOBAL u32x4_t *) (a.w0 + (static_cast<size_t>(n >> 4) * (K / 32) + w * KS + st) * 512 + l * 8);
+                        bv[t][g][st] = b;
                     } else {
                         bv[t][g][st] = *(const NAVI_GLOBAL u32x4_t *) (wr[t][g] + k);
                     }
@@ -209,13 +216,13 @@ __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int m = m0 + 16 * i + 4 * kq + r;
-                if (m < a.M) old[r] = a.y[PK ? pk_a(m, nb, a.ypk) : static_cast<size_t>(m) * a.ldy + nb];
+                if (m < a.M && mycol) old[r] = a.y[PK ? pk_a(m, nb, a.ypk) : static_cast<size_t>(m) * a.ldy + nb];
             }
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int mr = 16 * i + 4 * kq + r, m = m0 + mr;
-            if (m >= a.M) continue;
+            if (m >= a.M || !mycol) continue;
             const float sc = NORM ? rscale[mr] : 1.f;
             float *dst = a.y + (PK && EPI != EPI_PLAIN ? pk_a(m, nb, a.ypk) : static_cast<size_t>(m) * a.ldy + nb);
             if constexpr (EPI == EPI_PLAIN) {
@@ -314,10 +321,10 @@ void tile_rows(const float *src, int T, int H, float *x, hipStream_t s, uint32_t
     hipLaunchKernelGGL(k_tile_rows, dim3((T * (H / 4) + 255) / 256), dim3(256), 0, s, src, T, H, x, clear);
 }
 
-template <int MT, int EPI, bool NORM, int NWV, int KS, int CG>
+template <int MT, int EPI, bool NORM, int NWV, int KS, int CG, int CS = 1>
 void launch_pk(int M, int N, const RowArgs &ra, hipStream_t s) {
-    const dim3 grid(N / (16 * CG), (M + 16 * MT - 1) / (16 * MT));
-    hipLaunchKernelGGL((k_rows<MT, EPI, NORM, NWV, KS, CG, true>), grid, dim3(NWV * WAVE), 0, s, ra);
+    const dim3 grid(N / (16 * CG) * CS, (M + 16 * MT - 1) / (16 * MT));
+    hipLaunchKernelGGL((k_rows<MT, EPI, NORM, NWV, KS, CG, true, CS>), grid, dim3(NWV * WAVE), 0, s, ra);
 }
 
 // The projections of the multi-stream decode and of short prompts on the tile layouts (talker shapes: K 1024 into q|k|v and gate|up,
@@ -353,12 +360,14 @@ bool launch_rows_pk(int epi, bool norm, const float *A, int M, int K, const floa
     if (epi == EPI_RESID && K == 2048) {
         if (wide && M <= 96) launch_pk<1, EPI_RESID, false, 16, 4, 2>(M, N, ra, s);   // more blocks where they are few
         else if (wide) launch_pk<1, EPI_RESID, false, 16, 4, 4>(M, N, ra, s);
-        else launch_pk<1, EPI_RESID, false, 16, 4, 1>(M, N, ra, s);
+        else if (M <= 16) launch_pk<1, EPI_RESID, false, 16, 4, 1, 4>(M, N, ra, s);
+        else launch_pk<1, EPI_RESID, false, 16, 4, 1, 2>(M, N, ra, s);
         return true;
     }
     if (epi == EPI_RESID && K == 3072) {
         if (wide) launch_pk<1, EPI_RESID, false, 16, 6, 2>(M, N, ra, s);
-        else launch_pk<1, EPI_RESID, false, 16, 6, 1>(M, N, ra, s);
+        else if (M <= 16) launch_pk<1, EPI_RESID, false, 16, 6, 1, 4>(M, N, ra, s);
+        else launch_pk<1, EPI_RESID, false, 16, 6, 1, 2>(M, N, ra, s);
         return true;
     }
     return false;
