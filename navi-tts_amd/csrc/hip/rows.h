@@ -65,18 +65,19 @@ typedef _Float16 rhalf8 __attribute__((ext_vector_type(8)));
 // a.ypk); the same products in the same order, so the same bits as the row-major kernel.
 // CS > 1 (one column group): CS blocks share the 16 columns of a weight tile, each storing 16 / CS of them
 // and reading only those rows of the tile (the others' operands are zeros): the same sums, over more CUs.
-template <int MT, int EPI, bool NORM, int NWV, int KS, int CG = 1, bool PK = false, int CS = 1>
+template <int MT, int EPI, bool NORM, int NWV, int KS, int CG = 1, bool PK = false, int CS = 1, int RS = 1>
 __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
-    static_assert(CS == 1 || (CG == 1 && PK), "a split weight tile");
+    static_assert((CS == 1 && RS == 1) || (CG == 1 && MT == 1 && PK && !NORM), "split tiles");
     constexpr int NT = EPI == EPI_SWIGLU ? 2 : 1, K = 32 * KS * NWV;
     static_assert(CG * MT <= NWV, "one finishing wave per output tile");
     __shared__ f32x4_t red[NWV][NT][CG][MT][WAVE];
     __shared__ float ssq[NWV][MT][WAVE];
     __shared__ float rscale[MT * 16];
     const int w = static_cast<int>(threadIdx.x) / WAVE, l = static_cast<int>(threadIdx.x) & (WAVE - 1);
-    const int c = l & 15, kq = l >> 4, m0 = blockIdx.y * (MT * 16);
+    const int c = l & 15, kq = l >> 4, m0 = static_cast<int>(blockIdx.y) / RS * (MT * 16);
     const int cb = static_cast<int>(blockIdx.x) / CS;  // column block
     const int nb0 = cb * (16 * CG) + c;                // column of group 0; group g: nb0 + 16 g
+    auto myrow = [&](int r) { return RS == 1 || r / (16 / RS) == static_cast<int>(blockIdx.y) % RS; };
     const bool mycol = CS == 1 || c / (16 / CS) == static_cast<int>(blockIdx.x) % CS;
     auto wrow = [&](int n) {
         return n < a.n1 ? a.w0 + static_cast<size_t>(n) * K
@@ -111,13 +112,13 @@ __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
                 const int m = m0 + 16 * i + c;
-                if (PK && m < a.M) {
+                if (PK && m < a.M && myrow(c)) {
                     // lanes of a 16-row tile read one contiguous 1 KB when ars == 1 and aoff == 0
                     const int r = m * a.ars + a.aoff;
                     const NAVI_GLOBAL f32x4_t *p = (const NAVI_GLOBAL f32x4_t *) (a.a + (static_cast<size_t>(r >> 4) * (K / 32) + w * KS + st) * 512 + ((r & 15) + 16 * kq) * 4);
                     av[st][i][0] = p[0];
                     av[st][i][1] = p[64];
-                } else if (m < a.M) {
+                } else if (!PK && m < a.M) {
                     const NAVI_GLOBAL f32x4_t *p = (const NAVI_GLOBAL f32x4_t *) (a.a + static_cast<size_t>(m) * a.lda + k);
                     av[st][i][0] = p[0];
                     av[st][i][1] = p[1];
@@ -216,13 +217,13 @@ __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int m = m0 + 16 * i + 4 * kq + r;
-                if (m < a.M && mycol) old[r] = a.y[PK ? pk_a(m, nb, a.ypk) : static_cast<size_t>(m) * a.ldy + nb];
+                if (m < a.M && mycol && myrow(4 * kq + r)) old[r] = a.y[PK ? pk_a(m, nb, a.ypk) : static_cast<size_t>(m) * a.ldy + nb];
             }
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int mr = 16 * i + 4 * kq + r, m = m0 + mr;
-            if (m >= a.M || !mycol) continue;
+            if (m >= a.M || !mycol || !myrow(4 * kq + r)) continue;
             const float sc = NORM ? rscale[mr] : 1.f;
             float *dst = a.y + (PK && EPI != EPI_PLAIN ? pk_a(m, nb, a.ypk) : static_cast<size_t>(m) * a.ldy + nb);
             if constexpr (EPI == EPI_PLAIN) {
@@ -321,10 +322,10 @@ void tile_rows(const float *src, int T, int H, float *x, hipStream_t s, uint32_t
     hipLaunchKernelGGL(k_tile_rows, dim3((T * (H / 4) + 255) / 256), dim3(256), 0, s, src, T, H, x, clear);
 }
 
-template <int MT, int EPI, bool NORM, int NWV, int KS, int CG, int CS = 1>
+template <int MT, int EPI, bool NORM, int NWV, int KS, int CG, int CS = 1, int RS = 1>
 void launch_pk(int M, int N, const RowArgs &ra, hipStream_t s) {
-    const dim3 grid(N / (16 * CG) * CS, (M + 16 * MT - 1) / (16 * MT));
-    hipLaunchKernelGGL((k_rows<MT, EPI, NORM, NWV, KS, CG, true, CS>), grid, dim3(NWV * WAVE), 0, s, ra);
+    const dim3 grid(N / (16 * CG) * CS, (M + 16 * MT - 1) / (16 * MT) * RS);
+    hipLaunchKernelGGL((k_rows<MT, EPI, NORM, NWV, KS, CG, true, CS, RS>), grid, dim3(NWV * WAVE), 0, s, ra);
 }
 
 // The projections of the multi-stream decode and of short prompts on the tile layouts (talker shapes: K 1024 into q|k|v and gate|up,
@@ -346,6 +347,7 @@ bool launch_rows_pk(int epi, bool norm, const float *A, int M, int K, const floa
     // q|k|v and a whole-M tile for gate|up above (the sweep's best at 64 rows)
     if (epi == EPI_PLAIN && norm && K == 1024) {
         if (wide) launch_pk<1, EPI_PLAIN, true, 8, 4, 8>(M, N, ra, s);
+        else if (M > 16 && M <= 32 && N >= 4096) launch_pk<1, EPI_PLAIN, true, 8, 4, 2>(M, N, ra, s);
         else if (M <= 32) launch_pk<1, EPI_PLAIN, true, 8, 4, 1>(M, N, ra, s);
         else launch_pk<2, EPI_PLAIN, true, 8, 4, 1>(M, N, ra, s);
         return true;
@@ -361,13 +363,13 @@ bool launch_rows_pk(int epi, bool norm, const float *A, int M, int K, const floa
         if (wide && M <= 96) launch_pk<1, EPI_RESID, false, 16, 4, 2>(M, N, ra, s);   // more blocks where they are few
         else if (wide) launch_pk<1, EPI_RESID, false, 16, 4, 4>(M, N, ra, s);
         else if (M <= 16) launch_pk<1, EPI_RESID, false, 16, 4, 1, 4>(M, N, ra, s);
-        else launch_pk<1, EPI_RESID, false, 16, 4, 1, 2>(M, N, ra, s);
+        else launch_pk<1, EPI_RESID, false, 16, 4, 1, 1, 2>(M, N, ra, s);
         return true;
     }
     if (epi == EPI_RESID && K == 3072) {
         if (wide) launch_pk<1, EPI_RESID, false, 16, 6, 2>(M, N, ra, s);
         else if (M <= 16) launch_pk<1, EPI_RESID, false, 16, 6, 1, 4>(M, N, ra, s);
-        else launch_pk<1, EPI_RESID, false, 16, 6, 1, 2>(M, N, ra, s);
+        else launch_pk<1, EPI_RESID, false, 16, 6, 1, 1, 2>(M, N, ra, s);
         return true;
     }
     return false;
