@@ -366,16 +366,21 @@ __global__ void __launch_bounds__(BT) k_gather_rows(const uint16_t *table, const
     for (int i = threadIdx.x; i < width; i += BT) gst(dst + i, h2f(gld(src + i)));
 }
 
-// out[t] = A[ia[t]] + B[ib[t]] (+ spk on spk_row), entries < 0 absent, k_assemble_rows (talker.hip:27-41).
-__global__ void __launch_bounds__(BT) k_assemble_rows(const float *A, const float *B, const float *spk, const int32_t *ia,
-                                                      const int32_t *ib, int spk_row, int width, float *out) {
-    const int t = blockIdx.x, a_i = gld(ia + t), b_i = gld(ib + t);
+// Every row a prompt hands out in one launch (k_assemble_rows, talker.hip:27-41): row t is projected text
+// row rows[2 t] plus the codec embedding of id rows[2 t + 1] (none if < 0), plus the speaker on
+// spk_row; rows [0, n_pre) go to prefill, the next n_trail to trailing, the last one (a plain copy) to pad.
+__global__ void __launch_bounds__(BT) k_assemble_prompt(const float *proj, const uint16_t *codec_emb, const float *spk,
+                                                        const int32_t *rows, int spk_row, int n_pre, int n_trail, int width,
+                                                        float *prefill, float *trailing, float *pad) {
+    const int t = blockIdx.x, a_i = gld(rows + 2 * t), c_i = gld(rows + 2 * t + 1);
+    const bool is_pad = t == n_pre + n_trail;
+    float *out = is_pad ? pad : t < n_pre ? prefill + static_cast<size_t>(t) * width : trailing + static_cast<size_t>(t - n_pre) * width;
     for (int i = threadIdx.x; i < width; i += BT) {
-        float v = 0.f;
-        if (a_i >= 0) v += gld(A + static_cast<size_t>(a_i) * width + i);
-        if (b_i >= 0) v += gld(B + static_cast<size_t>(b_i) * width + i);
+        const float p = gld(proj + static_cast<size_t>(a_i) * width + i);
+        float v = is_pad ? p : 0.f + p;
+        if (c_i >= 0) v += h2f(gld(codec_emb + static_cast<size_t>(c_i) * width + i));
         if (t == spk_row) v += gld(spk + i);
-        gst(out + static_cast<size_t>(t) * width + i, v);
+        gst(out + i, v);
     }
 }
 
@@ -522,8 +527,11 @@ struct navi_talker {
     uint32_t *flag = nullptr;
     bool flag_set = false;             // whether a call may have left the flag set
     uint32_t *h_flag = nullptr;        // pinned host copy of flag, read back with the call's last sync
-    int32_t *d_ids = nullptr, *d_cids = nullptr, *d_ia = nullptr, *d_ib = nullptr, *d_ta = nullptr, *d_tb = nullptr;
-    float *text_rows = nullptr, *fc1_out = nullptr, *proj = nullptr, *codec_rows = nullptr, *spk = nullptr;
+    // a prompt's host data, staged in pinned memory and sent in one copy: the speaker [H] | text ids | the
+    // (text row, codec id) pairs of the rows to assemble
+    int32_t *d_stage = nullptr, *h_stage = nullptr;
+    size_t stage_words = 0;
+    float *text_rows = nullptr, *fc1_out = nullptr, *proj = nullptr;
     float *prefill = nullptr, *trailing = nullptr, *pad_row = nullptr, *hidden = nullptr, *logits = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double last_ms = 0;
@@ -547,6 +555,7 @@ struct navi_talker {
         if (ev0) (void) hipEventDestroy(ev0);
         if (ev1) (void) hipEventDestroy(ev1);
         if (h_flag) (void) hipHostFree(h_flag);
+        if (h_stage) (void) hipHostFree(h_stage);
         for (void *p : owned) (void) hipFree(p);
     }
 };
@@ -703,17 +712,11 @@ navi_status navi_talker_create(const navi_model_params *p, const navi_tensor_ref
     TALLOC(t->part, t->part_floats);
     TALLOC(t->invf, HD / 2);
     TALLOC(t->flag, 1);
-    TALLOC(t->d_ids, M);
-    TALLOC(t->d_cids, 16);
-    TALLOC(t->d_ia, M);
-    TALLOC(t->d_ib, M);
-    TALLOC(t->d_ta, M);
-    TALLOC(t->d_tb, M);
+    t->stage_words = t->H + M + 2 * (M + 16);
+    TALLOC(t->d_stage, t->stage_words);
     TALLOC(t->text_rows, M * t->TH);
     TALLOC(t->fc1_out, M * t->TH);
     TALLOC(t->proj, M * t->H);
-    TALLOC(t->codec_rows, 16 * t->H);
-    TALLOC(t->spk, t->H);
     TALLOC(t->prefill, M * t->H);
     TALLOC(t->trailing, M * t->H);
     TALLOC(t->pad_row, t->H);
@@ -754,6 +757,7 @@ navi_status navi_talker_create(const navi_model_params *p, const navi_tensor_ref
     hipLaunchKernelGGL(k_rotation, dim3(static_cast<unsigned>(M)), dim3(HD / 2), 0, s, t->invf, t->rot);
     if (hipEventCreate(&t->ev0) != hipSuccess || hipEventCreate(&t->ev1) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void **>(&t->h_flag), 64, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void **>(&t->h_stage), t->stage_words * 4, hipHostMallocDefault) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
         set_err(err, errlen, "talker: HIP setup failed");
         return fail(NAVI_ERR_HIP);
@@ -812,31 +816,35 @@ navi_status navi_talker_build_prompt(navi_talker *t, const int32_t *ids, int32_t
             set_err(err, errlen, "talker: codec control id %d outside the codec vocabulary", c);
             return NAVI_ERR_INVALID;
         }
-    // prefill: role rows, think rows (+ tts_pad), speaker (+ tts_pad), tts_bos + codec_pad, text[0] + codec_bos
-    std::vector<int32_t> ia, ib;
-    for (int r = 0; r < 3; ++r) { ia.push_back(r); ib.push_back(-1); }
-    for (int r = 0; r < n_think; ++r) { ia.push_back(i_pad); ib.push_back(r); }
-    const int spk_row = static_cast<int>(ia.size());
-    ia.push_back(i_pad); ib.push_back(-1);
-    ia.push_back(i_bos); ib.push_back(n_think);
-    ia.push_back(3); ib.push_back(n_think + 1);
-    // trailing: text[1:] then tts_eos
-    std::vector<int32_t> ta, tb;
-    for (int r = 1; r < n_text; ++r) { ta.push_back(3 + r); tb.push_back(-1); }
-    ta.push_back(i_eos); tb.push_back(-1);
-    const int n_pre = static_cast<int>(ia.size()), n_trail = static_cast<int>(ta.size());
+    // prefill: role rows, think rows (+ tts_pad), speaker (+ tts_pad), tts_bos + codec_pad, text[0] + codec_bos;
+    // trailing: text[1:] then tts_eos; then the tts_pad row itself
+    const int n_pre = 3 + n_think + 3, n_trail = n_text, spk_row = 3 + n_think;
+    float *spk = reinterpret_cast<float *>(t->h_stage);
+    int32_t *sid = t->h_stage + t->H, *row = sid + n_rows;
+    std::memcpy(spk, speaker, static_cast<size_t>(t->H) * 4);
+    std::memcpy(sid, tids.data(), tids.size() * 4);
+    int n_out = 0;
+    auto put = [&](int text, int codec) {
+        row[2 * n_out] = text;
+        row[2 * n_out + 1] = codec;
+        ++n_out;
+    };
+    for (int r = 0; r < 3; ++r) put(r, -1);
+    for (int r = 0; r < n_think; ++r) put(i_pad, cids[r]);
+    put(i_pad, -1);
+    put(i_bos, cids[n_think]);
+    put(3, cids[n_think + 1]);
+    for (int r = 1; r < n_text; ++r) put(3 + r, -1);
+    put(i_eos, -1);
+    put(i_pad, -1);
 
     hipStream_t s = device_state().stream;
-    NAVI_TRY_HIP(hipMemsetAsync(t->flag, 0, 4, s), err, errlen);
+    if (t->flag_set) NAVI_TRY_HIP(hipMemsetAsync(t->flag, 0, 4, s), err, errlen);
     t->flag_set = true;
-    NAVI_TRY_HIP(hipMemcpyAsync(t->d_ids, tids.data(), tids.size() * 4, hipMemcpyHostToDevice, s), err, errlen);
-    NAVI_TRY_HIP(hipMemcpyAsync(t->d_cids, cids.data(), cids.size() * 4, hipMemcpyHostToDevice, s), err, errlen);
-    NAVI_TRY_HIP(hipMemcpyAsync(t->spk, speaker, t->H * 4, hipMemcpyHostToDevice, s), err, errlen);
-    NAVI_TRY_HIP(hipMemcpyAsync(t->d_ia, ia.data(), ia.size() * 4, hipMemcpyHostToDevice, s), err, errlen);
-    NAVI_TRY_HIP(hipMemcpyAsync(t->d_ib, ib.data(), ib.size() * 4, hipMemcpyHostToDevice, s), err, errlen);
-    NAVI_TRY_HIP(hipMemcpyAsync(t->d_ta, ta.data(), ta.size() * 4, hipMemcpyHostToDevice, s), err, errlen);
-    NAVI_TRY_HIP(hipMemcpyAsync(t->d_tb, tb.data(), tb.size() * 4, hipMemcpyHostToDevice, s), err, errlen);
-    hipLaunchKernelGGL(k_gather_rows, dim3(n_rows), dim3(BT), 0, s, t->text_emb, t->d_ids, t->TH, t->text_rows);
+    NAVI_TRY_HIP(hipMemcpyAsync(t->d_stage, t->h_stage, (static_cast<size_t>(t->H) + n_rows + 2 * n_out) * 4, hipMemcpyHostToDevice, s),
+                 err, errlen);
+    const int32_t *d_ids = t->d_stage + t->H;
+    hipLaunchKernelGGL(k_gather_rows, dim3(n_rows), dim3(BT), 0, s, t->text_emb, d_ids, t->TH, t->text_rows);
     int S = pick_splits(n_rows, t->TH, t->TH);
     launch_partial(t->text_rows, t->TH, n_rows, t->fc1, t->TH, t->TH, S, t->part, t->TH, 0, t->flag, s);
     hipLaunchKernelGGL(k_finish_linear, dim3(n_rows), dim3(BT), 0, s, t->part, S, n_rows, t->TH, t->fc1_b, nullptr, 1,
@@ -845,14 +853,8 @@ navi_status navi_talker_build_prompt(navi_talker *t, const int32_t *ids, int32_t
     launch_partial(t->fc1_out, t->TH, n_rows, t->fc2, t->TH, t->H, S, t->part, t->H, 0, t->flag, s);
     hipLaunchKernelGGL(k_finish_linear, dim3(n_rows), dim3(BT), 0, s, t->part, S, n_rows, t->H, t->fc2_b, nullptr, 0,
                        t->proj, t->H);
-    hipLaunchKernelGGL(k_gather_rows, dim3(static_cast<unsigned>(cids.size())), dim3(BT), 0, s, t->codec_emb, t->d_cids,
-                       t->H, t->codec_rows);
-    hipLaunchKernelGGL(k_assemble_rows, dim3(n_pre), dim3(BT), 0, s, t->proj, t->codec_rows, t->spk, t->d_ia, t->d_ib,
-                       spk_row, t->H, t->prefill);
-    hipLaunchKernelGGL(k_assemble_rows, dim3(n_trail), dim3(BT), 0, s, t->proj, t->codec_rows, t->spk, t->d_ta, t->d_tb,
-                       -1, t->H, t->trailing);
-    NAVI_TRY_HIP(hipMemcpyAsync(t->pad_row, t->proj + static_cast<size_t>(i_pad) * t->H, t->H * 4,
-                                hipMemcpyDeviceToDevice, s), err, errlen);
+    hipLaunchKernelGGL(k_assemble_prompt, dim3(n_out), dim3(BT), 0, s, t->proj, t->codec_emb, reinterpret_cast<const float *>(t->d_stage),
+                       d_ids + n_rows, spk_row, n_pre, n_trail, t->H, t->prefill, t->trailing, t->pad_row);
     NAVI_TRY_HIP(hipGetLastError(), err, errlen);
     const navi_status st = check_flag(*t, "build_prompt", err, errlen);
     if (st != NAVI_OK) return st;
