@@ -375,15 +375,16 @@ __global__ void __launch_bounds__(256) k_split_rows(const float *src, const floa
 // running softmax of its own. Scores are computed transposed (K Q^T: lane l holds query row l % 16 and
 // keys 4 (l / 16) .. + 3 of each 16-key tile): the probabilities of a lane are its own MFMA operand for
 // V^T P^T (vf holds the keys in that order), split into f16 hi + lo as the queries are. The four
-// waves' sums meet in LDS at the end. Bound by the operand loads (16 KB per 32 keys and wave against
-// 64 MFMAs). Grid (kv groups, row tiles), the tiles with the most keys first; kv group g's blocks run
+// waves' sums meet in LDS at the end. The exponentials are the hardware's 2^x of the unscaled scores'
+// distance from the maximum (one rounding of the difference, one of its product with the scale): expf
+// took more instructions than everything else here. Grid (kv groups, row tiles), the tiles with the most keys first; kv group g's blocks run
 // on XCD g, whose L2 holds its keys and values.
 struct AttnArgs {
     const uint16_t *q, *kf, *vf;
     uint16_t *att;                    // split layout [T][nq 128]
     uint32_t *flag;
     int T, nq;
-    float scale;
+    float scale;                      // of the scores, times log2(e): the softmax is taken in powers of two
 };
 
 __global__ void __launch_bounds__(4 * WAVE, 2) k_attn_prompt(AttnArgs a) {
@@ -443,19 +444,19 @@ __global__ void __launch_bounds__(4 * WAVE, 2) k_attn_prompt(AttnArgs a) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int key = 32 * s + 16 * t + 4 * g + r;
-                    sc[h][t][r] = key <= row ? sc[h][t][r] * a.scale : -INFINITY;
+                    sc[h][t][r] = key <= row ? sc[h][t][r] : -INFINITY;
                     m = fmaxf(m, sc[h][t][r]);
                 }
             m = fmaxf(m, __shfl_xor(m, 16));
             m = fmaxf(m, __shfl_xor(m, 32));                 // finite: a step's first key is no later than any row
-            const float corr = expf(mx[h] - m);
+            const float corr = __builtin_amdgcn_exp2f((mx[h] - m) * a.scale);
             mx[h] = m;
             float ls = 0.f;
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float e = expf(sc[h][t][r] - m);
+                    const float e = __builtin_amdgcn_exp2f((sc[h][t][r] - m) * a.scale);
                     ls += e;
                     const _Float16 hi = static_cast<_Float16>(e);
                     ph[h][4 * t + r] = hi;
@@ -490,7 +491,7 @@ __global__ void __launch_bounds__(4 * WAVE, 2) k_attn_prompt(AttnArgs a) {
     float f[4], total = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        f[i] = expf(mb[i][h][c] - m);                        // 0 for a wave without keys
+        f[i] = __builtin_amdgcn_exp2f((mb[i][h][c] - m) * a.scale);   // 0 for a wave without keys
         total += f[i] * lb[i][h][c];
     }
     bool bad = false;

@@ -908,7 +908,7 @@ bool prefill_layers(navi_talker &t, int T, hipStream_t s) {
             b.nkv = t.NKV;
             gm::launch_qkv(b, s);
             hipLaunchKernelGGL(gm::k_attn_prompt, dim3(t.NKV, (T + 15) / 16), dim3(4 * WAVE), 0, s,
-                               gm::AttnArgs{half(t.q), t.kf, t.vf, half(t.att), t.flag, T, t.NQ, scale / w.q_scale});
+                               gm::AttnArgs{half(t.q), t.kf, t.vf, half(t.att), t.flag, T, t.NQ, static_cast<float>(1.4426950408889634 / (std::sqrt(static_cast<double>(HD)) * w.q_scale))});
             b = a;
             b.x = half(t.att);
             b.w = w.o_t;
