@@ -15,9 +15,9 @@
 //
 // What bounds them: the operand bytes into a CU (about 70 GB/s from L2, with the products switched
 // off as with them on), then the waits of the epilogue, which is why what it reads goes out before
-// the loop. 1001 rows, per layer: q|k|v 54.8 -> 30 us, gate|up 71.8 -> 34, o 26.7 -> 17, down 50.5 ->
-// 21.5, attention 124 -> 21.4; the prefill 9.22 -> 3.43 ms. 130 rows: 15.3 -> 10.6, 16.1 -> 10.7, 8.4
-// -> 8.4, 14.5 -> 10.6, 10.8 -> 8.5; 1.85 -> 1.37 ms. Sixteen-row blocks over whole-K (what these
+// the loop. 1001 rows, per layer: q|k|v 54.8 -> 26.5 us, gate|up 71.8 -> 29, o 26.7 -> 15.3, down 50.5 ->
+// 20.4, attention 124 -> 17.8; the prefill 9.23 -> 3.19 ms. 130 rows: 15.3 -> 10.6, 16.1 -> 10.7, 8.4
+// -> 8.4, 14.5 -> 10.6, 10.8 -> 8.1; 1.85 -> 1.34 ms. Sixteen-row blocks over whole-K (what these
 // replaced) read every weight once per 16 rows. Measured and left out: the same tiles staged in LDS by
 // eight waves (q|k|v at 1001 rows 25 us, but 21 us at 80 rows and gate|up 35), the loop unrolled over
 // all of K (half as fast again: its code does not stay in the instruction cache), three and more steps
@@ -248,14 +248,17 @@ struct Epilogue {
     }
 };
 
-// NW waves, each PER steps of 32 of K = 32 NW PER, with ST load slots (ST - 1 steps in flight).
-template <int MT, int NT, int EPI, int NW, int PER, int ST, int WPS>
+// NW waves, each PER steps of 32 of K = 32 NW PER, with ST load slots (ST - 1 steps in flight). ST = 1: two
+// slots for X and one for W, whose fragments are asked for again as soon as their products are out,
+// half a step's registers less than ST = 2: two blocks of a 64 x 128 tile share a CU, and one's
+// epilogue runs under the other's loop. The waves' tiles are exchanged MX 16-row tiles at a time.
+template <int MT, int NT, int EPI, int NW, int PER, int ST, int WPS, int MX = MT>
 __global__ void __launch_bounds__(NW * WAVE, WPS) k_gemm(GemmArgs a) {
     static_assert(EPI != G_QKV || NT == 8, "a block of the q|k|v projection owns one head");
     static_assert(NT % 2 == 0, "as many up columns as gate columns; 32 columns per partial sum of squares");
-    static_assert(MT <= NW && PER % ST == 0, "a wave finishes one 16-row tile; whole rounds of the load slots");
+    static_assert(MT <= NW && PER % ST == 0 && MT % MX == 0, "a wave finishes one 16-row tile; whole rounds of the load slots");
     constexpr int STEPS = NW * PER;
-    __shared__ f32x4_t red[MT][NW - 1][NT][WAVE];
+    __shared__ f32x4_t red[MX][NW - 1][NT][WAVE];
     const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6), l = static_cast<int>(threadIdx.x) & 63;
     const int g = l >> 4, mtiles = (a.M + 15) >> 4, nrow = (mtiles + MT - 1) / MT;
     int col, row;
@@ -274,15 +277,19 @@ __global__ void __launch_bounds__(NW * WAVE, WPS) k_gemm(GemmArgs a) {
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[i][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    u32x4_t fx[ST][MT][2], fw[ST][NT];
+    u32x4_t fx[ST > 1 ? ST : 2][MT][2], fw[ST][NT];
     const uint32_t lo = static_cast<uint32_t>(l) * 8;
-    auto load = [&](int slot, int s) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) fw[slot][t] = *(const NAVI_GLOBAL u32x4_t *) (wb[t] + s * 512 + lo);
+    auto load_w = [&](int slot, int t, int s) { fw[slot][t] = *(const NAVI_GLOBAL u32x4_t *) (wb[t] + s * 512 + lo); };
+    auto load_x = [&](int slot, int s) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int p = 0; p < 2; ++p) fx[slot][i][p] = *(const NAVI_GLOBAL u32x4_t *) (xb[i] + s * 1024 + p * 512 + lo);
+    };
+    auto load = [&](int slot, int s) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) load_w(slot, t, s);
+        load_x(slot, s);
     };
     auto mma = [&](int slot) {
 #pragma unroll
@@ -301,49 +308,84 @@ __global__ void __launch_bounds__(NW * WAVE, WPS) k_gemm(GemmArgs a) {
     };
 #pragma unroll
     for (int u = 0; u < ST - 1; ++u) load(u, u);
+    if constexpr (ST == 1) load(0, 0);
     const int m = (row * MT + w) * 16 + (l & 15);           // the row this lane finishes (w < MT)
     Epilogue<NT, EPI> end;
     end.load(a, col, m, g);
     if constexpr (MT == 1) end.load_head(a, col, m, g);
     __builtin_amdgcn_sched_barrier(0);
-    int s = 0;
-#pragma unroll 1
-    for (; s < PER - ST; s += ST)
-#pragma unroll
-        for (int u = 0; u < ST; ++u) {
-            load((u + ST - 1) % ST, s + u + ST - 1);
-            __builtin_amdgcn_sched_barrier(0);
-            mma(u);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-    for (int u = 0; u < ST; ++u) {
-        if (u == 0) load(ST - 1, PER - 1);
-        mma(u);
-    }
-    if constexpr (MT > 1) end.load_head(a, col, m, g);
-    // wave o finishes 16-row tile o
-#pragma unroll
-    for (int o = 0; o < MT; ++o)
-        if (o != w) {
-            const int src = w < o ? w : w - 1;
-#pragma unroll
-            for (int t = 0; t < NT; ++t) red[o][src][t][l] = acc[o][t];
-        }
-    __syncthreads();
-    if (w >= MT) return;
-    // in wave order whichever wave finishes the tile; one uniform branch per wave, constant indices
-    f32x4_t v[NT];
-#pragma unroll
-    for (int o = 0; o < MT; ++o)
-        if (o == w)
+    if constexpr (ST == 1) {
+        auto step = [&](int xs, int s, bool more) {
+            if (more) load_x(xs ^ 1, s + 1);
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                f32x4_t sum = o == 0 ? acc[o][t] : red[o][0][t][l];
+                ghalf8 wv;
+                __builtin_memcpy(&wv, &fw[0][t], 16);
 #pragma unroll
-                for (int u = 1; u < NW; ++u) sum += u == o ? acc[o][t] : red[o][u < o ? u : u - 1][t][l];
-                v[t] = sum;
+                for (int p = 0; p < 2; ++p)
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) {
+                        ghalf8 xv;
+                        __builtin_memcpy(&xv, &fx[xs][i][p], 16);
+                        acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xv, acc[i][t], 0, 0, 0);
+                    }
+                if (more) load_w(0, t, s + 1);
+                __builtin_amdgcn_sched_barrier(0);
             }
+        };
+        static_assert(ST > 1 || PER % 2 == 0, "two X slots");
+#pragma unroll 1
+        for (int s = 0; s < PER - 2; s += 2) {
+            step(0, s, true);
+            step(1, s + 1, true);
+        }
+        step(0, PER - 2, true);
+        step(1, PER - 1, false);
+    } else {
+        int s = 0;
+#pragma unroll 1
+        for (; s < PER - ST; s += ST)
+#pragma unroll
+            for (int u = 0; u < ST; ++u) {
+                load((u + ST - 1) % ST, s + u + ST - 1);
+                __builtin_amdgcn_sched_barrier(0);
+                mma(u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+        for (int u = 0; u < ST; ++u) {
+            if (u == 0) load(ST - 1, PER - 1);
+            mma(u);
+        }
+    }
+    if constexpr (MT > 1 && ST > 1) end.load_head(a, col, m, g);
+    // wave o finishes 16-row tile o; sums in wave order whichever wave it is; uniform branches and constant
+    // indices (an indexed register array would go to memory)
+    f32x4_t v[NT];
+#pragma unroll
+    for (int j = 0; j < MT; j += MX) {
+        if (j) __syncthreads();                             // the previous tiles' readers are done
+#pragma unroll
+        for (int o = j; o < j + MX; ++o)
+            if (o != w) {
+                const int src = w < o ? w : w - 1;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) red[o - j][src][t][l] = acc[o][t];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int o = j; o < j + MX; ++o)
+            if (o == w)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    f32x4_t sum = o == 0 ? acc[o][t] : red[o - j][0][t][l];
+#pragma unroll
+                    for (int u = 1; u < NW; ++u) sum += u == o ? acc[o][t] : red[o - j][u < o ? u : u - 1][t][l];
+                    v[t] = sum;
+                }
+    }
+    if (w >= MT) return;
+    if constexpr (MT > 1 && ST == 1) end.load_head(a, col, m, g);
     bool bad = false;
     end.finish(a, col, m, mtiles, g, v, bad);
     if (bad) gst(a.flag, 1u);
@@ -506,23 +548,26 @@ __global__ void __launch_bounds__(4 * WAVE, 2) k_attn_prompt(AttnArgs a) {
     if (bad) gst(a.flag, 1u);
 }
 
-template <int MT, int NT, int EPI, int NW, int PER, int ST, int WPS>
+template <int MT, int NT, int EPI, int NW, int PER, int ST, int WPS, int MX = MT>
 void launch_gemm(const GemmArgs &a, hipStream_t s) {
     const int ncol = EPI == G_SWIGLU ? a.N / (8 * NT) : a.N / (16 * NT), nrow = ((a.M + 15) / 16 + MT - 1) / MT;
-    hipLaunchKernelGGL((k_gemm<MT, NT, EPI, NW, PER, ST, WPS>), dim3(ncol * nrow), dim3(NW * WAVE), 0, s, a);
+    hipLaunchKernelGGL((k_gemm<MT, NT, EPI, NW, PER, ST, WPS, MX>), dim3(ncol * nrow), dim3(NW * WAVE), 0, s, a);
 }
 
 // The talker's shapes (K 1024 into q|k|v and gate|up, 2048 into o, 3072 into down; N 4096, 2 x 3072,
 // 1024, 1024). A launch takes about as long as its longest block as long as every block has a CU of
 // its own, so the tile is the smallest that still gives at most 256 blocks: a block's time is its
 // operand bytes (about 70 GB/s from L2 into one CU, whatever the other CUs do), and a block more
-// than CUs is a second round.
+// than CUs is a second round. Above 512 rows no tile gives that: there the one-slot form, two blocks to a
+// CU (768 rows: q|k|v 26 -> 23 us, gate|up 30 -> 23; 1001 rows 27.5 -> 26.5 and 30.5 -> 29).
 void launch_qkv(const GemmArgs &a, hipStream_t s) {
     const int mt = (a.M + 15) / 16;
     if (mt <= 8) launch_gemm<1, 8, G_QKV, 4, 8, 2, 2>(a, s);
     else if (mt <= 16) launch_gemm<2, 8, G_QKV, 4, 8, 2, 1>(a, s);
     else if (mt <= 24) launch_gemm<3, 8, G_QKV, 4, 8, 2, 1>(a, s);
-    else launch_gemm<4, 8, G_QKV, 4, 8, 2, 1>(a, s);
+    else if (mt <= 32) launch_gemm<4, 8, G_QKV, 4, 8, 2, 1>(a, s);
+    else if (mt <= 48) launch_gemm<2, 8, G_QKV, 4, 8, 1, 2>(a, s);
+    else launch_gemm<4, 8, G_QKV, 4, 8, 1, 2, 2>(a, s);
 }
 void launch_gate_up(const GemmArgs &a, hipStream_t s) {
     const int mt = (a.M + 15) / 16;
@@ -530,7 +575,8 @@ void launch_gate_up(const GemmArgs &a, hipStream_t s) {
     else if (mt <= 8) launch_gemm<2, 6, G_SWIGLU, 4, 8, 2, 2>(a, s);
     else if (mt <= 10) launch_gemm<2, 8, G_SWIGLU, 4, 8, 2, 1>(a, s);
     else if (mt <= 16) launch_gemm<4, 6, G_SWIGLU, 4, 8, 2, 1>(a, s);
-    else launch_gemm<4, 12, G_SWIGLU, 4, 8, 2, 1>(a, s);
+    else if (mt <= 32) launch_gemm<4, 12, G_SWIGLU, 4, 8, 2, 1>(a, s);
+    else launch_gemm<4, 6, G_SWIGLU, 4, 8, 1, 2, 2>(a, s);
 }
 // STEPS = K / 32
 template <int STEPS>
@@ -539,7 +585,7 @@ void launch_resid(const GemmArgs &a, hipStream_t s) {
     if (mt <= 8) launch_gemm<1, 2, G_RESID, 8, STEPS / 8, 4, 2>(a, s);
     else if (mt <= 16) launch_gemm<2, 2, G_RESID, 8, STEPS / 8, 2, 2>(a, s);
     else if (mt <= 32) launch_gemm<2, 4, G_RESID, 8, STEPS / 8, 2, 2>(a, s);
-    else launch_gemm<4, 4, G_RESID, 8, STEPS / 8, 2, 2>(a, s);
+    else launch_gemm<4, 4, G_RESID, 8, STEPS / 8, 1, 2>(a, s);
 }
 
 } // namespace

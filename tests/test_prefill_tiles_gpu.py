@@ -59,10 +59,10 @@ def _rows(T):
     return np.random.default_rng(T).standard_normal((T, 1024)).astype(np.float32)
 
 
-# the last row count of one tile choice and the first of the next: gate|up 80, 128, 160, 256; q|k|v
-# 128, 256, 384; o and down 128, 256, 512 (65, 256, 257, 512 and 513 are in test_prefill_gpu.py);
-# 96: an even number of 16-row tiles with no ragged row
-@pytest.mark.parametrize("T", [66, 80, 81, 96, 128, 129, 160, 161, 384, 385])
+# the last row count of one tile choice and the first of the next: gate|up 80, 128, 160, 256, 512; q|k|v
+# 128, 256, 384, 512, 768; o and down 128, 256, 512 (65, 256, 257, 512 and 513 are in
+# test_prefill_gpu.py); 96: an even number of 16-row tiles with no ragged row
+@pytest.mark.parametrize("T", [66, 80, 81, 96, 128, 129, 160, 161, 384, 385, 768, 769])
 def test_prefill_tile_edges_match_oracle(side, T):
     side.check(_rows(T))
 
