@@ -1419,8 +1419,8 @@ navi_status frame_kv(navi_frame *f, const navi_kv_view *kv, int n_past_min, int 
     for (int l = 0; l < kv->n_layer; ++l) same = same && f->kv_host[0][l] == kv->k[l] && f->kv_host[1][l] == kv->v[l];
     if (!same) {
         for (int l = 0; l < kv->n_layer; ++l) { f->kv_host[0][l] = kv->k[l]; f->kv_host[1][l] = kv->v[l]; }
-        // not waited for: the frames behind it are, before the table can change again
-        if (hipMemcpyAsync(f->kv_dev, f->kv_host, sizeof(f->kv_host), hipMemcpyHostToDevice, device_state().stream) != hipSuccess) {
+        if (hipMemcpyAsync(f->kv_dev, f->kv_host, sizeof(f->kv_host), hipMemcpyHostToDevice, device_state().stream) != hipSuccess ||
+            hipStreamSynchronize(device_state().stream) != hipSuccess) {
             msg = "frame: KV pointer upload failed";
             return NAVI_ERR_HIP;
         }
