@@ -17,8 +17,8 @@
 //  * Attentive statistics pooling: in [x | mean | std] the mean and std columns are the same at
 //    every time step, so their part of asp.tdnn is folded into a per-channel bias (one GEMV) and
 //    the conv runs over the 1536 x channels only: the [T][4608] concatenation is never built.
-//  * Time reductions (SE mean, pooling statistics, softmax over time) run 16 channels x 16 time
-//    slices per block, summed in a fixed order: the same bits every run. k=1 convs with few
+//  * Time reductions (SE mean, pooling statistics with their softmax over time) run 16 channels x 64
+//    time slices per block, summed in a fixed order: the same bits every run. k=1 convs with few
 //    output tiles (the SE and fc GEMVs, attentive pooling's 128-channel conv) split their input
 //    channels over blocks; the partial sums are added in split order.
 #include "conv.h"
@@ -38,30 +38,54 @@ namespace spk {
 using namespace cv;
 
 constexpr int C = 512, R = 64, SCALE = 8, SEC = 128, MFA = 1536, ASP = 128;
-constexpr int NCH = 16, NPART = BT / NCH;     // time reductions: 16 channels x 16 time slices per block
 
 // ---- time reductions ---------------------------------------------------------------------
-// Thread (q, c) sums rows t = q, q + 16, ... of channel c; the 16 slice sums are added in slice
-// order by one thread: fixed association, the same bits every run.
+// 16 channels x 64 time slices per block: thread (q, c) takes rows t = q, q + 64, ... of channel c in
+// order; the slice sums are added four by four in the wave, then in wave order: fixed association,
+// the same bits every run. They are bound by the latency of their row loads, so a thread asks for RU
+// rows at once (all of its rows up to 1024 frames, 10.9 s) and the statistics keep the first RU in
+// registers for their later passes; longer audio reads the rest again.
+constexpr int NCH = 16, RT = 1024, NPART = RT / NCH, RU = 16;
+static_assert(C % NCH == 0 && MFA % NCH == 0, "whole blocks of channels");
 
-__device__ __forceinline__ float slice_total(float (&red)[NPART][NCH], int cl) {
-    float s = red[0][cl];
+// rows t0 + NPART k of a channel (x: row 0's element), zero past T
+__device__ __forceinline__ void load_rows(const float *x, int t0, int T, int ld, float (&v)[RU]) {
 #pragma unroll
-    for (int q = 1; q < NPART; ++q) s += red[q][cl];
-    return s;
+    for (int k = 0; k < RU; ++k) {
+        const int t = t0 + k * NPART;
+        v[k] = t < T ? gld(x + static_cast<size_t>(t) * ld) : 0.f;
+    }
 }
 
-// mean over time of x[t][c] (ld ldx), c < C_: out[c]
-__global__ void __launch_bounds__(BT) k_time_mean(const float *x, int T, int C_, int ldx, float *out) {
-    __shared__ float red[NPART][NCH];
-    const int cl = threadIdx.x % NCH, c = blockIdx.x * NCH + cl, q = threadIdx.x / NCH;
-    float s = 0.f;
-    if (c < C_)
-#pragma unroll 4
-        for (int t = q; t < T; t += NPART) s += gld(x + static_cast<size_t>(t) * ldx + c);
-    red[q][cl] = s;
+// op over the time slices of each channel, in every thread
+template <class F>
+__device__ __forceinline__ float slices(float v, float (&red)[RT / WAVE][NCH], F op) {
+    v = op(v, __shfl_xor(v, 16));
+    v = op(v, __shfl_xor(v, 32));
+    __syncthreads();                                        // the previous reduction's readers are done
+    const int cl = threadIdx.x % NCH;
+    if ((threadIdx.x & (WAVE - 1)) < NCH) red[threadIdx.x / WAVE][cl] = v;
     __syncthreads();
-    if (q == 0 && c < C_) gst(out + c, slice_total(red, cl) / static_cast<float>(T));
+    float s = red[0][cl];
+#pragma unroll
+    for (int i = 1; i < RT / WAVE; ++i) s = op(s, red[i][cl]);
+    return s;
+}
+__device__ __forceinline__ float add(float a, float b) { return a + b; }
+
+// mean over time of x[t][c] (ld ldx): out[c]. 512 channels, 937 rows: 6.8 -> 4.0 us.
+__global__ void __launch_bounds__(RT) k_time_mean(const float *x, int T, int ldx, float *out) {
+    __shared__ float red[RT / WAVE][NCH];
+    const int c = blockIdx.x * NCH + threadIdx.x % NCH, q = threadIdx.x / NCH;
+    float s = 0.f;
+    for (int t0 = q; t0 < T; t0 += RU * NPART) {
+        float v[RU];
+        load_rows(x + c, t0, T, ldx, v);
+#pragma unroll
+        for (int k = 0; k < RU; ++k) s += v[k];
+    }
+    s = slices(s, red, add);
+    if (q == 0) gst(out + c, s / static_cast<float>(T));
 }
 
 // y[t][c] = b[t][c] * g[c] + r[t][c]   (squeeze-excitation scale + the block's residual)
@@ -73,87 +97,50 @@ __global__ void __launch_bounds__(BT) k_scale_add(const float *b, int ldb, const
     gst(y + static_cast<size_t>(t) * ldy + c, gld(b + static_cast<size_t>(t) * ldb + c) * gld(g + c) + gld(r + static_cast<size_t>(t) * ldr + c));
 }
 
-// Per channel c < C_: mean and std over time with weights w[t][c] (uniform 1/T when w is null):
-// out[c] = sum w x, out[C_ + c] = sqrt(max(sum w (x - mean)^2, 1e-12)) (k_weighted_stats, speaker.hip:92-107).
-__global__ void __launch_bounds__(BT) k_stats(const float *x, const float *w, int T, int C_, int ld, float *out) {
-    __shared__ float red[NPART][NCH];
-    __shared__ float mean[NCH];
-    const int cl = threadIdx.x % NCH, c = blockIdx.x * NCH + cl, q = threadIdx.x / NCH;
-    const float u = 1.f / static_cast<float>(T);
-    float s = 0.f;
-    if (c < C_)
-#pragma unroll 4
-        for (int t = q; t < T; t += NPART) {
-            const size_t o = static_cast<size_t>(t) * ld + c;
-            s = fmaf(w ? gld(w + o) : u, gld(x + o), s);
+// Per channel c < C_: mean and std over time of x[t][c] with weights w[t][c], uniform 1 / T (SOFT = 0) or the
+// softmax over time of the logits a[t][c]: out[c] = sum w x, out[C_ + c] = sqrt(max(sum w (x - mean)^2,
+// 1e-12)) (k_weighted_stats, speaker.hip:92-107). The weights are not stored: a softmax kernel and a
+// statistics kernel that read them back, four rows asked for at a time, took 21.2 + 12.5 us at 1536 x 937,
+// this one 10.8; the uniform case 12.4 -> 4.8 (10 s of audio 460 -> 423 us).
+template <int SOFT>
+__global__ void __launch_bounds__(RT) k_stats(const float *x, const float *a, int T, int C_, int ld, float *out) {
+    __shared__ float red[RT / WAVE][NCH];
+    const int c = blockIdx.x * NCH + threadIdx.x % NCH, q = threadIdx.x / NCH;
+    float xv[RU], av[RU] = {};
+    if (SOFT) load_rows(a + c, q, T, ld, av);
+    load_rows(x + c, q, T, ld, xv);
+    // f(x, a) over the thread's rows
+    auto each = [&](auto f) {
+#pragma unroll
+        for (int k = 0; k < RU; ++k)
+            if (q + k * NPART < T) f(xv[k], av[k]);
+        for (int t0 = q + RU * NPART; t0 < T; t0 += RU * NPART) {
+            float x2[RU], a2[RU] = {};
+            if (SOFT) load_rows(a + c, t0, T, ld, a2);
+            load_rows(x + c, t0, T, ld, x2);
+#pragma unroll
+            for (int k = 0; k < RU; ++k)
+                if (t0 + k * NPART < T) f(x2[k], a2[k]);
         }
-    red[q][cl] = s;
-    __syncthreads();
-    if (q == 0) mean[cl] = slice_total(red, cl);
-    __syncthreads();
-    const float m = mean[cl];
-    float v = 0.f;
-    if (c < C_)
-#pragma unroll 4
-        for (int t = q; t < T; t += NPART) {
-            const size_t o = static_cast<size_t>(t) * ld + c;
-            const float d = gld(x + o) - m;
-            v = fmaf(w ? gld(w + o) : u, d * d, v);
-        }
-    __syncthreads();
-    red[q][cl] = v;
-    __syncthreads();
-    if (q == 0 && c < C_) {
-        gst(out + c, m);
-        gst(out + C_ + c, sqrtf(fmaxf(slice_total(red, cl), 1e-12f)));
+    };
+    float mx = -INFINITY, inv = 1.f / static_cast<float>(T);
+    if (SOFT) {
+        each([&](float, float l) { mx = fmaxf(mx, l); });
+        mx = slices(mx, red, [](float l, float r) { return fmaxf(l, r); });
+        float t = 0.f;
+        each([&](float, float l) { t += expf(l - mx); });
+        inv = 1.f / slices(t, red, add);
     }
-}
-
-// softmax over time per channel, in place: a[t][c] (ld ld), c < C_
-__global__ void __launch_bounds__(BT) k_time_softmax(float *a, int T, int C_, int ld) {
-    __shared__ float red[NPART][NCH];
-    __shared__ float tot[NCH];
-    const int cl = threadIdx.x % NCH, c = blockIdx.x * NCH + cl, q = threadIdx.x / NCH;
-    float m = -INFINITY;
-    if (c < C_)
-#pragma unroll 4
-        for (int t = q; t < T; t += NPART) m = fmaxf(m, gld(a + static_cast<size_t>(t) * ld + c));
-    red[q][cl] = m;
-    __syncthreads();
+    auto weight = [&](float l) { return SOFT ? expf(l - mx) * inv : inv; };
+    float s = 0.f, v = 0.f;
+    each([&](float e, float l) { s = fmaf(weight(l), e, s); });
+    const float m = slices(s, red, add);
+    each([&](float e, float l) { v = fmaf(weight(l), (e - m) * (e - m), v); });
+    v = slices(v, red, add);
     if (q == 0) {
-        float mx = red[0][cl];
-#pragma unroll
-        for (int i = 1; i < NPART; ++i) mx = fmaxf(mx, red[i][cl]);
-        tot[cl] = mx;
+        gst(out + c, m);
+        gst(out + C_ + c, sqrtf(fmaxf(v, 1e-12f)));
     }
-    __syncthreads();
-    const float mx = tot[cl];
-    float s = 0.f;
-    if (c < C_)
-#pragma unroll 4
-        for (int t = q; t < T; t += NPART) s += expf(gld(a + static_cast<size_t>(t) * ld + c) - mx);
-    __syncthreads();
-    red[q][cl] = s;
-    __syncthreads();
-    if (q == 0) tot[cl] = slice_total(red, cl);
-    __syncthreads();
-    const float inv = 1.f / tot[cl];
-    // in place: four rows' loads go out before their stores (a load after a store to the same
-    // array would wait for it)
-    if (c < C_)
-        for (int t0 = q; t0 < T; t0 += 4 * NPART) {
-            float v[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int t = t0 + k * NPART;
-                v[k] = t < T ? gld(a + static_cast<size_t>(t) * ld + c) : 0.f;
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int t = t0 + k * NPART;
-                if (t < T) gst(a + static_cast<size_t>(t) * ld + c, expf(v[k] - mx) * inv);
-            }
-        }
 }
 
 // The attentive pooling's constant columns folded into a bias: out[co] = b[co] + sum_i
@@ -408,7 +395,7 @@ struct navi_speaker {
     // SpeakerEncoder::Impl::run (speaker.hip:175-220) over the T mel rows in `mel`.
     navi_status run(int T, char *err, size_t errlen) {
         hipStream_t s = device_state().stream;
-        const unsigned tb = static_cast<unsigned>((C + NCH - 1) / NCH), tm = static_cast<unsigned>((MFA + NCH - 1) / NCH);
+        const unsigned tb = C / NCH, tm = MFA / NCH;
 #define SP_TRY(x)                                                                               \
         do {                                                                                    \
             const navi_status st_ = (x);                                                        \
@@ -429,7 +416,7 @@ struct navi_speaker {
             SP_TRY(conv(bk.tdnn2, PRO_NONE, EPI_RELU, c, T, C, b, C, err, errlen));
             // squeeze-excitation on the time mean, then out = b * gate + the block input, written
             // into this block's slice of the MFA input (which is also the next block's input)
-            hipLaunchKernelGGL(k_time_mean, dim3(tb), dim3(BT), 0, s, b, T, C, C, mean);
+            hipLaunchKernelGGL(k_time_mean, dim3(tb), dim3(RT), 0, s, b, T, C, mean);
             SP_TRY(conv(bk.se1, PRO_NONE, EPI_RELU, mean, 1, C, g, SEC, err, errlen));
             SP_TRY(conv(bk.se2, PRO_NONE, EPI_SIGMOID, g, 1, SEC, gse, C, err, errlen));
             float *out = cat3 + bi * C;
@@ -441,12 +428,11 @@ struct navi_speaker {
         }
         SP_TRY(conv(mfa, PRO_NONE, EPI_RELU, cat3, T, MFA, att, MFA, err, errlen));
         // attentive statistics pooling
-        hipLaunchKernelGGL(k_stats, dim3(tm), dim3(BT), 0, s, att, nullptr, T, MFA, MFA, stats);
+        hipLaunchKernelGGL(k_stats<0>, dim3(tm), dim3(RT), 0, s, att, nullptr, T, MFA, MFA, stats);
         hipLaunchKernelGGL(k_asp_bias, dim3(ASP), dim3(BT), 0, s, asp_w, asp_b, stats, bias2);
         SP_TRY(conv(asp_x, PRO_NONE, EPI_RELU_TANH, att, T, MFA, g2, ASP, err, errlen, nullptr, bias2));
         SP_TRY(conv(asp_conv, PRO_NONE, EPI_BIAS, g2, T, ASP, attw, MFA, err, errlen));
-        hipLaunchKernelGGL(k_time_softmax, dim3(tm), dim3(BT), 0, s, attw, T, MFA, MFA);
-        hipLaunchKernelGGL(k_stats, dim3(tm), dim3(BT), 0, s, att, attw, T, MFA, MFA, pooled);
+        hipLaunchKernelGGL(k_stats<1>, dim3(tm), dim3(RT), 0, s, att, attw, T, MFA, MFA, pooled);
         SP_TRY(conv(fc, PRO_NONE, EPI_BIAS, pooled, 1, 2 * MFA, emb, p.enc_dim, err, errlen));
 #undef SP_TRY
         NAVI_TRY_HIP(hipGetLastError(), err, errlen);
