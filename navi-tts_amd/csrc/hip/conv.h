@@ -17,8 +17,8 @@ constexpr int LDW = CCH + 8;             // padded LDS row (halves)
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 
-// Prologues (applied to the input as it is staged): SILU_GATE silu(x[ci]) * x[Cin + ci]; ADD2 x + x2.
-enum Pro { PRO_NONE = 0, PRO_SILU_GATE = 2, PRO_ADD2 = 3 };
+// Prologue (applied to the input as it is staged): SILU_GATE silu(x[ci]) * x[Cin + ci].
+enum Pro { PRO_NONE = 0, PRO_SILU_GATE = 2 };
 // Epilogues after the bias: RELU_TANH is tanh(max(v, 0)); PARTIAL stores split-K partial sums.
 enum Epi { EPI_BIAS = 0, EPI_GELU = 1, EPI_RESIDUAL = 2, EPI_SCALE_RESIDUAL = 3, EPI_CLAMP = 4, EPI_PARTIAL = 5,
            EPI_RELU = 6, EPI_SIGMOID = 7, EPI_RELU_TANH = 8 };
@@ -38,7 +38,6 @@ struct ConvArgs {
     const float *za, *zb;
     float *part;           // EPI_PARTIAL: [splits][T * phases][Cout] partial sums, no bias
     uint32_t *flag;        // set when a (prologue-applied) activation is outside the f16 range
-    const float *x2;       // PRO_ADD2: second input, same layout as x
     // When set: the causal history the next chunk reads (the last (K-1) dil rows of [hist ; x]),
     // written by this launch into the other buffer of the conv's history pair.
     float *hnext;
@@ -251,7 +250,7 @@ __global__ void __launch_bounds__(BT) k_conv_mfma(ConvArgs a) {
     // and the next chunk's go out before this chunk's MFMAs, so no load waits on another.
     constexpr int Q4 = CCH / 4, RPI = BT / Q4;               // float4s per staged row, rows per item step
     constexpr int IT = (WROWS + RPI - 1) / RPI;
-    constexpr bool TWO = PRO == PRO_SILU_GATE || PRO == PRO_ADD2;   // a second operand per element
+    constexpr bool TWO = PRO == PRO_SILU_GATE;              // a second operand per element
     static_assert(BT % Q4 == 0, "every item step covers whole rows");
     const int c4 = (static_cast<int>(threadIdx.x) % Q4) * 4, rr0 = static_cast<int>(threadIdx.x) / Q4;
     int off[IT];
@@ -286,15 +285,13 @@ __global__ void __launch_bounds__(BT) k_conv_mfma(ConvArgs a) {
         const int ci = ci0 + c4;
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
-            // plain values, then one store each: filled in under branches the arrays were kept in scratch
-            // memory for K = 3 with a second operand (the speaker encoder's Res2Net chain, 10 s of
-            // audio 496 -> 460 us)
+            // plain values, then one store each: filled in under branches such arrays can end up in
+            // scratch memory (they did at K = 3 with a second operand)
             const bool x = in && ((xm >> it) & 1u), h = in && ((hm >> it) & 1u);
             f32x4_t v = {0.f, 0.f, 0.f, 0.f}, w = {0.f, 0.f, 0.f, 0.f};
             if (x) v = *(const NAVI_GLOBAL f32x4_t *) (a.x + off[it] + ci);
             else if (h) v = *(const NAVI_GLOBAL f32x4_t *) (a.hist + off[it] + ci);
             if (PRO == PRO_SILU_GATE && x) w = *(const NAVI_GLOBAL f32x4_t *) (a.x + off[it] + a.Cin + ci);
-            if (PRO == PRO_ADD2 && x) w = *(const NAVI_GLOBAL f32x4_t *) (a.x2 + off[it] + ci);
             av[it] = v;
             if (TWO) au[it] = w;
         }
@@ -318,7 +315,6 @@ __global__ void __launch_bounds__(BT) k_conv_mfma(ConvArgs a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = silu(v[e]) * au[it][e];
             }
-            if (PRO == PRO_ADD2) v += au[it];
             half4v h, o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {

@@ -9,10 +9,10 @@
 //    on the host (the reference's static SpeakerEncoder::mel, in double); navi_speaker_embed on
 //    the device, one block per frame (k_logmel: FFT in LDS, also in double), so a clone uploads
 //    audio, not a spectrogram, and no host loop sits on its path.
-//  * Every conv (block 0 k5, the SE-Res2Net tdnn / dilated k3 / squeeze-excitation convs, MFA,
+//  * Every conv (block 0 k5, the SE-Res2Net tdnn / squeeze-excitation convs, MFA,
 //    attentive pooling, fc) is conv.h's implicit GEMM on the matrix cores with "same" reflect
-//    padding; ReLU, sigmoid and tanh(ReLU) are its epilogues, the Res2Net "slice + previous
-//    output" input its ADD2 prologue. Each block writes its output straight into its slice of
+//    padding; ReLU, sigmoid and tanh(ReLU) are its epilogues. A block's Res2Net chain of seven
+//    small convs is one launch (k_res2net). Each block writes its output straight into its slice of
 //    the [T][1536] MFA input, which is also the next block's input (no copies).
 //  * Attentive statistics pooling: in [x | mean | std] the mean and std columns are the same at
 //    every time step, so their part of asp.tdnn is folded into a per-channel bias (one GEMV) and
@@ -49,9 +49,10 @@ constexpr int NCH = 16, RT = 1024, NPART = RT / NCH, RU = 16;
 static_assert(C % NCH == 0 && MFA % NCH == 0, "whole blocks of channels");
 
 // rows t0 + NPART k of a channel (x: row 0's element), zero past T
-__device__ __forceinline__ void load_rows(const float *x, int t0, int T, int ld, float (&v)[RU]) {
+template <int N>
+__device__ __forceinline__ void load_rows(const float *x, int t0, int T, int ld, float (&v)[N]) {
 #pragma unroll
-    for (int k = 0; k < RU; ++k) {
+    for (int k = 0; k < N; ++k) {
         const int t = t0 + k * NPART;
         v[k] = t < T ? gld(x + static_cast<size_t>(t) * ld) : 0.f;
     }
@@ -88,6 +89,150 @@ __global__ void __launch_bounds__(RT) k_time_mean(const float *x, int T, int ldx
     if (q == 0) gst(out + c, s / static_cast<float>(T));
 }
 
+// The Res2Net chain of one block: slice 0 of b passes to c, slice i = ReLU(conv_i(slice i of b + slice i -
+// 1 of c)), seven k3 convs over 64 channels, "same" with reflect padding. A block owns RB rows and
+// computes the whole chain for them: conv i on the rows that the later ones' taps reach, (7 - i) dil more
+// on either side (at most 64 rows: eight waves, two 16 x 16 tiles each), its output going into LDS as
+// the next one's input. The halo's products are done 2.5 times over; what bounds it is the latency of
+// the chain, and seven launches and a copy for a few rows each were 44 us (937 rows), this one
+// 16.5 (10 s of audio 423 -> 374 us). Per output the sums run as in k_conv_mfma: taps, 32-channel steps, hi then lo. Weights in
+// fragment order (k_tile_res): read 64 B per column and by sixteen waves, one tile each, the L1's
+// look-ups took 21 us.
+constexpr int RB = 16, RDIL = 4, RW = RB + 2 * (SCALE - 1) * RDIL, RWT = 512;   // RW: rows of the widest window
+static_assert(RB + 2 * (SCALE - 2) * RDIL <= 64 && R == 64 && RWT == 8 * WAVE, "four 16-row tiles by four column tiles");
+
+// A conv's weight [R][R][3] -> the B fragments [column tile][tap][32-channel step][lane][8]
+__global__ void k_tile_res(const uint16_t *w, uint16_t *out) {
+    const int i = static_cast<int>(blockIdx.x) * BT + static_cast<int>(threadIdx.x);
+    if (i >= R * R * 3) return;
+    const int e = i & 7, l = (i >> 3) & 63, f = i >> 9, s = f & 1, j = (f >> 1) % 3, n = f / 6;
+    gst(out + i, gld(w + ((16 * n + (l & 15)) * R + 32 * s + 8 * (l >> 4) + e) * 3 + j));
+}
+
+struct ResArgs {
+    const float *b;                       // [T][C]
+    float *c;                             // [T][C]
+    const uint16_t *w;                    // [SCALE - 1] tiled weights
+    const float *bias;                    // [SCALE - 1][R]
+    uint32_t *flag;
+    int T, dil;                           // 2 <= dil <= RDIL, dil < T
+};
+
+__global__ void __launch_bounds__(RWT) k_res2net(ResArgs a) {
+    __shared__ __align__(16) _Float16 hi[2][RW][LDW];
+    __shared__ __align__(16) _Float16 lo[2][RW][LDW];
+    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, co = 16 * (wv & 3) + (l & 15);
+    const int t0 = static_cast<int>(blockIdx.x) * RB, base = t0 - (SCALE - 1) * a.dil, rows = RB + 2 * (SCALE - 1) * a.dil;
+    bool bad = false;
+    auto split = [&](float v, _Float16 &h, _Float16 &o) {
+        bad |= !(fabsf(v) < 65504.f);
+        h = static_cast<_Float16>(v);
+        o = static_cast<_Float16>(v - static_cast<float>(h));
+    };
+    u32x4_t bq[3][2];
+    float bias;
+    auto load_w = [&](int i) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+                bq[j][s] = *(const NAVI_GLOBAL u32x4_t *) (a.w + (((i * 4 + (wv & 3)) * 3 + j) * 2 + s) * 512 + l * 8);
+        bias = gld(a.bias + i * R + co);
+    };
+    // waits for LDS only: the weights in flight and the stores go on across it
+    auto barrier = [&] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    load_w(0);
+    {   // slice 1 of the window, slice 0 of the block's own rows
+        const int c4 = (static_cast<int>(threadIdx.x) & 15) * 4, r0 = static_cast<int>(threadIdx.x) >> 4;
+        constexpr int IT = (RW + RWT / 16 - 1) / (RWT / 16);
+        f32x4_t v[IT], p = {0.f, 0.f, 0.f, 0.f};
+        const bool own = r0 < RB && t0 + r0 < a.T;
+        if (own) p = ld4(a.b + static_cast<size_t>(t0 + r0) * C + c4);
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int r = r0 + it * (RWT / 16), t = base + r;
+            f32x4_t e = {0.f, 0.f, 0.f, 0.f};
+            if (r < rows && t >= 0 && t < a.T) e = ld4(a.b + static_cast<size_t>(t) * C + R + c4);
+            v[it] = e;
+        }
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int r = r0 + it * (RWT / 16);
+            if (r >= rows) continue;
+            half4v h, o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                _Float16 he, oe;
+                split(v[it][e], he, oe);
+                h[e] = he;
+                o[e] = oe;
+            }
+            *reinterpret_cast<half4v *>(&hi[0][r][c4]) = h;
+            *reinterpret_cast<half4v *>(&lo[0][r][c4]) = o;
+        }
+        if (own) st4(a.c + static_cast<size_t>(t0 + r0) * C + c4, p);
+    }
+    barrier();
+#pragma unroll 1
+    for (int i = 1; i < SCALE; ++i) {
+        const int reach = (SCALE - 1 - i) * a.dil, cur = (i - 1) & 1, need = RB + 2 * reach;
+        const int tile = t0 - reach + 16 * (wv >> 2);       // rows tile .. + 15 and tile + 32 .. + 47
+        const bool two = 16 * (wv >> 2) + 32 < need;
+        if (16 * (wv >> 2) < need) {
+            float x[2][4];                                  // slice i + 1 at this conv's rows
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = tile + 32 * m + 4 * (l >> 4) + r;
+                    x[m][r] = gld(a.b + static_cast<size_t>(min(max(t, 0), a.T - 1)) * C + min(i + 1, SCALE - 1) * R + co);
+                }
+            f32x4_t acc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                int row[2];
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    int t = tile + 32 * m + (l & 15) + (j - 1) * a.dil;
+                    t = t < 0 ? -t : t >= a.T ? 2 * (a.T - 1) - t : t;
+                    row[m] = min(max(t - base, 0), rows - 1);   // rows past the reach are computed and dropped
+                }
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    half8v b;
+                    __builtin_memcpy(&b, &bq[j][s], 16);
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) {
+                        if (m == 1 && !two) continue;
+                        const half8v h = *reinterpret_cast<const half8v *>(&hi[cur][row[m]][s * 32 + (l >> 4) * 8]);
+                        const half8v o = *reinterpret_cast<const half8v *>(&lo[cur][row[m]][s * 32 + (l >> 4) * 8]);
+                        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(h, b, acc[m], 0, 0, 0);
+                        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o, b, acc[m], 0, 0, 0);
+                    }
+                }
+            }
+            const float bi = bias;
+            if (i + 1 < SCALE) load_w(i);
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = tile + 32 * m + 4 * (l >> 4) + r;
+                    if (t < 0 || t >= a.T || t >= t0 + RB + reach) continue;
+                    const float v = fmaxf(acc[m][r] + bi, 0.f);
+                    if (t >= t0 && t < t0 + RB) gst(a.c + static_cast<size_t>(t) * C + i * R + co, v);
+                    if (i + 1 < SCALE) split(x[m][r] + v, hi[cur ^ 1][t - base][co], lo[cur ^ 1][t - base][co]);
+                }
+        }
+        barrier();
+    }
+    if (bad) gst(a.flag, 1u);
+}
+
 // y[t][c] = b[t][c] * g[c] + r[t][c]   (squeeze-excitation scale + the block's residual)
 __global__ void __launch_bounds__(BT) k_scale_add(const float *b, int ldb, const float *g, const float *r, int ldr, int T,
                                                   float *y, int ldy) {
@@ -109,33 +254,34 @@ __global__ void __launch_bounds__(RT) k_stats(const float *x, const float *a, in
     float xv[RU], av[RU] = {};
     if (SOFT) load_rows(a + c, q, T, ld, av);
     load_rows(x + c, q, T, ld, xv);
-    // f(x, a) over the thread's rows
+    // f(x, a, whether a is one that stays in its register) over the thread's rows
     auto each = [&](auto f) {
 #pragma unroll
         for (int k = 0; k < RU; ++k)
-            if (q + k * NPART < T) f(xv[k], av[k]);
-        for (int t0 = q + RU * NPART; t0 < T; t0 += RU * NPART) {
-            float x2[RU], a2[RU] = {};
+            if (q + k * NPART < T) f(xv[k], av[k], true);
+        constexpr int N = RU / 2;                           // with RU the softmax's registers spill
+        for (int t0 = q + RU * NPART; t0 < T; t0 += N * NPART) {
+            float x2[N], a2[N] = {};
             if (SOFT) load_rows(a + c, t0, T, ld, a2);
             load_rows(x + c, t0, T, ld, x2);
 #pragma unroll
-            for (int k = 0; k < RU; ++k)
-                if (t0 + k * NPART < T) f(x2[k], a2[k]);
+            for (int k = 0; k < N; ++k)
+                if (t0 + k * NPART < T) f(x2[k], a2[k], false);
         }
     };
     float mx = -INFINITY, inv = 1.f / static_cast<float>(T);
     if (SOFT) {
-        each([&](float, float l) { mx = fmaxf(mx, l); });
+        each([&](float, float l, bool) { mx = fmaxf(mx, l); });
         mx = slices(mx, red, [](float l, float r) { return fmaxf(l, r); });
         float t = 0.f;
-        each([&](float, float l) { t += expf(l - mx); });
+        each([&](float, float &l, bool) { t += l = expf(l - mx); });
         inv = 1.f / slices(t, red, add);
     }
-    auto weight = [&](float l) { return SOFT ? expf(l - mx) * inv : inv; };
+    auto weight = [&](float l, bool kept) { return SOFT ? (kept ? l : expf(l - mx)) * inv : inv; };
     float s = 0.f, v = 0.f;
-    each([&](float e, float l) { s = fmaf(weight(l), e, s); });
+    each([&](float e, float l, bool kept) { s = fmaf(weight(l, kept), e, s); });
     const float m = slices(s, red, add);
-    each([&](float e, float l) { v = fmaf(weight(l), (e - m) * (e - m), v); });
+    each([&](float e, float l, bool kept) { v = fmaf(weight(l, kept), (e - m) * (e - m), v); });
     v = slices(v, red, add);
     if (q == 0) {
         gst(out + c, m);
@@ -297,7 +443,6 @@ void launch_spk(const ConvArgs &a, int pro, int epi, dim3 grid, hipStream_t s) {
         hipLaunchKernelGGL((k_conv_mfma<MT, K, P_, E_>), grid, dim3(BT), 0, s, a);              \
         return;                                                                                 \
     }
-    if constexpr (K == 3) NAVI_SPK(PRO_ADD2, EPI_RELU)
     NAVI_SPK(PRO_NONE, EPI_RELU)
     if constexpr (K == 1) {
         NAVI_SPK(PRO_NONE, EPI_PARTIAL)
@@ -315,7 +460,10 @@ struct navi_speaker {
     int max_frames = 0;
     SConv block0, mfa, asp_x, asp_conv, fc;
     struct Block {
-        SConv tdnn1, res[SCALE - 1], tdnn2, se1, se2;
+        SConv tdnn1, tdnn2, se1, se2;
+        uint16_t *res_w = nullptr;            // the Res2Net chain's weights (k_tile_res) and biases
+        float *res_b = nullptr;               // [SCALE - 1][R], one after the other
+        int dil = 0;
     } blocks[3];
     const uint16_t *asp_w = nullptr;          // asp.tdnn as stored [ASP][3 MFA][1] (its mean/std columns)
     const float *asp_b = nullptr;
@@ -349,11 +497,11 @@ struct navi_speaker {
         for (void *v : owned) (void) hipFree(v);
     }
 
-    // "same" reflect-padded conv over T rows: x [T][ldx] -> y [T][ldy] (x2: the ADD2 input, ld ldx)
+    // "same" reflect-padded conv over T rows: x [T][ldx] -> y [T][ldy]
     navi_status conv(const SConv &cv, int pro, int epi, const float *x, int T, int ldx, float *y, int ldy, char *err,
-                     size_t errlen, const float *x2 = nullptr, const float *bias = nullptr) {
+                     size_t errlen, const float *bias = nullptr) {
         ConvArgs ca{};
-        ca.x = x; ca.x2 = x2; ca.w = cv.w; ca.bias = bias ? bias : cv.bias; ca.y = y; ca.flag = flag;
+        ca.x = x; ca.w = cv.w; ca.bias = bias ? bias : cv.bias; ca.y = y; ca.flag = flag;
         ca.ldx = ldx; ca.ldy = ldy; ca.T = T; ca.Cin = cv.Cin; ca.Cout = cv.Cout; ca.dil = cv.dil; ca.phases = 1;
         ca.cps = cv.Cin; ca.lpad = (cv.K - 1) * cv.dil / 2; ca.reflect = 1;
         // 16-row tiles unless that already gives the chip two blocks per CU
@@ -380,8 +528,6 @@ struct navi_speaker {
         switch (cv.K * 10 + mt) {
         case 11: launch_spk<1, 1>(ca, pro, epi, grid, s); break;
         case 14: launch_spk<4, 1>(ca, pro, epi, grid, s); break;
-        case 31: launch_spk<1, 3>(ca, pro, epi, grid, s); break;
-        case 34: launch_spk<4, 3>(ca, pro, epi, grid, s); break;
         case 51: launch_spk<1, 5>(ca, pro, epi, grid, s); break;
         case 54: launch_spk<4, 5>(ca, pro, epi, grid, s); break;
         default:
@@ -408,11 +554,9 @@ struct navi_speaker {
             Block &bk = blocks[bi];
             SP_TRY(conv(bk.tdnn1, PRO_NONE, EPI_RELU, in, T, ldin, b, C, err, errlen));
             // Res2Net: slice 0 passes, slice 1 = conv(slice 1), slice i = conv(slice i + out i-1)
-            NAVI_TRY_HIP(hipMemcpy2DAsync(c, C * sizeof(float), b, C * sizeof(float), R * sizeof(float), T,
-                                          hipMemcpyDeviceToDevice, s), err, errlen);
-            for (int i = 1; i < SCALE; ++i)
-                SP_TRY(conv(bk.res[i - 1], i == 1 ? PRO_NONE : PRO_ADD2, EPI_RELU, b + i * R, T, C, c + i * R, C, err, errlen,
-                            i == 1 ? nullptr : c + (i - 1) * R));
+            ResArgs ra{};
+            ra.b = b; ra.c = c; ra.flag = flag; ra.T = T; ra.dil = bk.dil; ra.w = bk.res_w; ra.bias = bk.res_b;
+            hipLaunchKernelGGL(k_res2net, dim3(static_cast<unsigned>((T + RB - 1) / RB)), dim3(RWT), 0, s, ra);
             SP_TRY(conv(bk.tdnn2, PRO_NONE, EPI_RELU, c, T, C, b, C, err, errlen));
             // squeeze-excitation on the time mean, then out = b * gate + the block input, written
             // into this block's slice of the MFA input (which is also the next block's input)
@@ -430,7 +574,7 @@ struct navi_speaker {
         // attentive statistics pooling
         hipLaunchKernelGGL(k_stats<0>, dim3(tm), dim3(RT), 0, s, att, nullptr, T, MFA, MFA, stats);
         hipLaunchKernelGGL(k_asp_bias, dim3(ASP), dim3(BT), 0, s, asp_w, asp_b, stats, bias2);
-        SP_TRY(conv(asp_x, PRO_NONE, EPI_RELU_TANH, att, T, MFA, g2, ASP, err, errlen, nullptr, bias2));
+        SP_TRY(conv(asp_x, PRO_NONE, EPI_RELU_TANH, att, T, MFA, g2, ASP, err, errlen, bias2));
         SP_TRY(conv(asp_conv, PRO_NONE, EPI_BIAS, g2, T, ASP, attw, MFA, err, errlen));
         hipLaunchKernelGGL(k_stats<1>, dim3(tm), dim3(RT), 0, s, att, attw, T, MFA, MFA, pooled);
         SP_TRY(conv(fc, PRO_NONE, EPI_BIAS, pooled, 1, 2 * MFA, emb, p.enc_dim, err, errlen));
@@ -612,7 +756,23 @@ navi_status navi_speaker_create(const navi_speaker_params *p, const navi_tensor_
         const std::string bp = S + "blocks." + std::to_string(b + 1) + ".";
         navi_speaker::Block &bk = h->blocks[b];
         SB(bp + "tdnn1.conv", C, C, 1, 1, bk.tdnn1);
-        for (int r = 0; r < SCALE - 1; ++r) SB(bp + "res2net_block.blocks." + std::to_string(r) + ".conv", R, R, 3, dils[b], bk.res[r]);
+        bk.dil = dils[b];
+        if ((st = h->alloc(bk.res_w, static_cast<size_t>(SCALE - 1) * R * R * 3, err, errlen)) != NAVI_OK ||
+            (st = h->alloc(bk.res_b, static_cast<size_t>(SCALE - 1) * R, err, errlen)) != NAVI_OK)
+            return fail(st);
+        for (int r = 0; r < SCALE - 1; ++r) {
+            const std::string name = bp + "res2net_block.blocks." + std::to_string(r) + ".conv";
+            const void *w = nullptr, *bias = nullptr;
+            if ((st = tensor(name + ".weight", NAVI_DT_F16, R, R, 3, w)) != NAVI_OK ||
+                (st = tensor(name + ".bias", NAVI_DT_F32, R, 0, 0, bias)) != NAVI_OK)
+                return fail(st);
+            hipLaunchKernelGGL(k_tile_res, dim3((R * R * 3 + BT - 1) / BT), dim3(BT), 0, s, static_cast<const uint16_t *>(w),
+                               bk.res_w + r * R * R * 3);
+            if (hipMemcpyAsync(bk.res_b + r * R, bias, R * sizeof(float), hipMemcpyDeviceToDevice, s) != hipSuccess) {
+                set_err(err, errlen, "speaker: bias copy failed");
+                return fail(NAVI_ERR_HIP);
+            }
+        }
         SB(bp + "tdnn2.conv", C, C, 1, 1, bk.tdnn2);
         SB(bp + "se_block.conv1", C, SEC, 1, 1, bk.se1);
         SB(bp + "se_block.conv2", SEC, C, 1, 1, bk.se2);
