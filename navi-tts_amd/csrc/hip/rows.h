@@ -65,6 +65,7 @@ typedef _Float16 rhalf8 __attribute__((ext_vector_type(8)));
 // a.ypk); the same products in the same order, so the same bits as the row-major kernel.
 // CS > 1 (one column group): CS blocks share the 16 columns of a weight tile, each storing 16 / CS of them
 // and reading only those rows of the tile (the others' operands are zeros): the same sums, over more CUs.
+// RS > 1: the same with the rows of a 16-row tile of A, RS blocks each finishing 16 / RS of them.
 template <int MT, int EPI, bool NORM, int NWV, int KS, int CG = 1, bool PK = false, int CS = 1, int RS = 1>
 __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
     static_assert((CS == 1 && RS == 1) || (CG == 1 && MT == 1 && PK && !NORM), "split tiles");
@@ -332,7 +333,11 @@ void launch_pk(int M, int N, const RowArgs &ra, hipStream_t s) {
 // 2048 into o, 3072 into down). A: [M][K] tiled; W: one [N][K] tiled matrix (q|k|v and gate|up
 // stacked); y: PLAIN row-major [M][ldy], SWIGLU ([M][F]) and RESID ([M][N]) tiled. Tile shapes from a
 // sweep at 10 and 130 rows (weights streamed from HBM): above 64 rows 16-row tiles with 8 (q|k|v),
-// 4 (gate|up, o) or 2 (down) column groups per block; up to 64 rows the one-group kernels. Every
+// 4 (gate|up, o) or 2 (down) column groups per block; up to 64 rows the one-group kernels, except
+// q|k|v at 17-32 rows, where two groups halve the reads of the second row tile. o and down have 64 column
+// tiles, a quarter of the CUs: up to 16 rows four blocks share each (a 10-row prompt 1.07 -> 1.03 ms),
+// up to 64 two blocks share each row tile (in place of two that share the columns and all read the rows,
+// with q|k|v's two groups: 32 streams 4.51 -> 4.43 ms a step). Every
 // shape keeps the row-major kernels' split of K over the waves, so the outputs are theirs bit for
 // bit (gate|up over 16 waves x 2 steps measured 0.7 us faster at 130 rows, with other bits).
 // false: a shape these kernels do not take.
