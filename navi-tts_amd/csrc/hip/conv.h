@@ -79,9 +79,16 @@ __device__ __forceinline__ float sin2_reduce(float u) {
     const float n = rintf(u * 0.318309873f);
     return fmaf(-n, -8.74227766e-8f, fmaf(-n, 3.14159274f, u));
 }
+// A pass leaves less than 2^-51 of an argument whose multiple of pi has more than 53 bits (2.8e16 on): three
+// bring every finite float into the polynomial's range. The phase holds up to about 2^80.
 __device__ __forceinline__ float sin2_reduce_wide(float u) {
-    const double m = rint(static_cast<double>(u) * 0.3183098861837907);
-    return static_cast<float>(fma(-m, 1.2246467991473532e-16, fma(-m, 3.141592653589793, static_cast<double>(u))));
+    double r = static_cast<double>(u);
+#pragma unroll 1
+    for (int pass = 0; pass < 3; ++pass) {
+        const double m = rint(r * 0.3183098861837907);
+        r = fma(-m, 1.2246467991473532e-16, fma(-m, 3.141592653589793, r));
+    }
+    return static_cast<float>(r);
 }
 
 // v + zb sin^2(za v) for N values of one channel: one branch for all of them, their chains interleaved.

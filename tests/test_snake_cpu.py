@@ -4,6 +4,7 @@ that of its last product allow about two units of 2^-24 each way, 2.5e-7; the re
 of r (half a unit of 1.6, times a slope of at most 1).
 """
 import re
+from fractions import Fraction
 from pathlib import Path
 
 import numpy as np
@@ -45,15 +46,28 @@ def test_sin2_f32_reduction(scale):
     assert np.allclose(got[small], want[small], rtol=5e-7, atol=0)
 
 
-@pytest.mark.parametrize("scale", [2.0 ** 20, 1e9, 1e13])
+def _wide(u):
+    """One argument of sin2_reduce_wide: three passes, their fma sums exact before they are rounded."""
+    r = float(u)
+    for _ in range(3):
+        m = Fraction(float(np.rint(np.float64(r) * 0.3183098861837907)))
+        t = float(Fraction(r) - m * Fraction(3.141592653589793))
+        r = float(Fraction(t) - m * Fraction(1.2246467991473532e-16))
+    return F(r)
+
+
+# 64-bit sin holds its phase over all of these; past 2.8e16 one pass alone would leave the polynomial's range
+@pytest.mark.parametrize("scale", [2.0 ** 20, 1e9, 1e13, 2e16, 1e17, 1e20, 1e23])
 def test_sin2_wide_reduction(scale):
-    u = (np.random.default_rng(2).uniform(1, 4, 100000) * scale).astype(F).astype(np.float64)
-    m = np.rint(u * 0.3183098861837907)
-    # the products exact, as the device's fma has them: in integers of 2^-102
-    hi, lo = 3.141592653589793, 1.2246467991473532e-16
-    from fractions import Fraction
-    idx = np.random.default_rng(3).integers(0, u.size, 300)
-    r = np.array([float(Fraction(float(u[i])) - Fraction(m[i]) * Fraction(hi) - Fraction(m[i]) * Fraction(lo)) for i in idx]).astype(F)
+    u = (np.random.default_rng(2).uniform(1, 4, 300) * scale).astype(F)
+    r = np.array([_wide(x) for x in u])
     assert np.abs(r).max() < 1.64
-    want = np.array([np.sin(float(u[i])) ** 2 for i in idx])
+    want = np.sin(u.astype(np.float64)) ** 2
     assert np.abs(_poly(r) - want).max() < 3e-7
+
+
+@pytest.mark.parametrize("u", [1e30, -3.4028234e38])
+def test_sin2_wide_reduction_is_bounded(u):
+    """Past the phase's reach the value is some sin^2 all the same."""
+    r = _wide(F(u))
+    assert abs(r) < 1.64 and 0 <= _poly(np.array([r]))[0] <= 1 + 3e-7
