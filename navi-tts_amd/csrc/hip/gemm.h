@@ -15,13 +15,13 @@
 //
 // What bounds them: the operand bytes into a CU (about 70 GB/s from L2, with the products switched
 // off as with them on), then the waits of the epilogue, which is why what it reads goes out before
-// the loop. 1001 rows, per layer: q|k|v 54.8 -> 26.5 us, gate|up 71.8 -> 29, o 26.7 -> 15.3, down 50.5 ->
-// 20.4, attention 124 -> 17.8; the prefill 9.23 -> 3.19 ms. 130 rows: 15.3 -> 10.6, 16.1 -> 10.7, 8.4
+// the loop. 1001 rows, per layer: q|k|v 54.8 -> 32 us, gate|up 71.8 -> 30, o 26.7 -> 16.4, down 50.5 ->
+// 21.2, attention 124 -> 17.0; the prefill 9.23 -> 3.31 ms. 130 rows: 15.3 -> 10.6, 16.1 -> 10.7, 8.4
 // -> 8.4, 14.5 -> 10.6, 10.8 -> 8.1; 1.85 -> 1.34 ms. Sixteen-row blocks over whole-K (what these
 // replaced) read every weight once per 16 rows. Measured and left out: the same tiles staged in LDS by
 // eight waves (q|k|v at 1001 rows 25 us, but 21 us at 80 rows and gate|up 35), the loop unrolled over
 // all of K (half as fast again: its code does not stay in the instruction cache), three and more steps
-// in flight (no faster), hi and lo products in accumulators of their own (+3 %, no closer to 64 bits).
+// in flight (no faster), hi and lo products in accumulators of their own (+3 %).
 #pragma once
 
 #include "rows.h"
@@ -250,14 +250,24 @@ struct Epilogue {
 
 // NW waves, each PER steps of 32 of K = 32 NW PER, with ST load slots (ST - 1 steps in flight). ST = 1: two
 // slots for X and one for W, whose fragments are asked for again as soon as their products are out,
-// half a step's registers less than ST = 2: two blocks of a 64 x 128 tile share a CU, and one's
-// epilogue runs under the other's loop. The waves' tiles are exchanged MX 16-row tiles at a time.
+// half a step's registers less than ST = 2: two blocks share a CU, and one's epilogue runs under the
+// other's loop. The waves' tiles are exchanged MX 16-row tiles at a time.
+//
+// A step's products start from zero (lo, then hi) and are added to the tile's sums by the vector units.
+// Chained on the sums in the matrix unit, every product is cut to the last bit of a sum that grows with
+// K: mean over twelve prompts of 100 rows, the first layer's keys and values then lie 9.1e-6 and 8.5e-6 from
+// 64 bits, like this 7.4e-6 and 7.2e-6 (the row kernels' half as long chains: 7.3e-6 and 8.8e-6), the final
+// hidden state 1.16e-4 and 9.9e-5 (1.25e-4). It costs nothing up to 300 rows and 4 % of the prefill at 1001. The
+// two largest gate|up tiles have no registers left for it and chain (CHAIN): their error reaches the keys and values
+// only through the residual stream (without it 768 rows take 2.98 ms instead of 2.79, the second
+// layer's keys and values at the same distance).
 template <int MT, int NT, int EPI, int NW, int PER, int ST, int WPS, int MX = MT>
 __global__ void __launch_bounds__(NW * WAVE, WPS) k_gemm(GemmArgs a) {
     static_assert(EPI != G_QKV || NT == 8, "a block of the q|k|v projection owns one head");
     static_assert(NT % 2 == 0, "as many up columns as gate columns; 32 columns per partial sum of squares");
     static_assert(MT <= NW && PER % ST == 0 && MT % MX == 0, "a wave finishes one 16-row tile; whole rounds of the load slots");
     constexpr int STEPS = NW * PER;
+    constexpr bool CHAIN = MT * NT * (ST == 1 ? 2 : 1) >= 48;   // 64 x 192, and 64 x 96 at half the registers: they would spill
     __shared__ f32x4_t red[MX][NW - 1][NT][WAVE];
     const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6), l = static_cast<int>(threadIdx.x) & 63;
     const int g = l >> 4, mtiles = (a.M + 15) >> 4, nrow = (mtiles + MT - 1) / MT;
@@ -291,20 +301,33 @@ __global__ void __launch_bounds__(NW * WAVE, WPS) k_gemm(GemmArgs a) {
         for (int t = 0; t < NT; ++t) load_w(slot, t, s);
         load_x(slot, s);
     };
+    // a step's lo (p = 1), then hi products: from zero into part, which add() adds to the tile's sums, or (CHAIN)
+    // straight onto them
+    auto product = [&](f32x4_t &part, f32x4_t &sum, const ghalf8 &wv, const ghalf8 &xv, int p) {
+        if constexpr (CHAIN) sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xv, sum, 0, 0, 0);
+        else part = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xv, p ? f32x4_t{0.f, 0.f, 0.f, 0.f} : part, 0, 0, 0);
+    };
+    auto add = [&](f32x4_t &sum, const f32x4_t &part) {
+        if constexpr (!CHAIN) sum += part;
+    };
     auto mma = [&](int slot) {
 #pragma unroll
-        for (int p = 0; p < 2; ++p)
+        for (int i = 0; i < MT; ++i) {
+            f32x4_t part[NT];
 #pragma unroll
-            for (int i = 0; i < MT; ++i) {
+            for (int p = 1; p >= 0; --p) {
                 ghalf8 xv;
                 __builtin_memcpy(&xv, &fx[slot][i][p], 16);
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     ghalf8 wv;
                     __builtin_memcpy(&wv, &fw[slot][t], 16);
-                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xv, acc[i][t], 0, 0, 0);
+                    product(part[t], acc[i][t], wv, xv, p);
                 }
             }
+#pragma unroll
+            for (int t = 0; t < NT; ++t) add(acc[i][t], part[t]);
+        }
     };
 #pragma unroll
     for (int u = 0; u < ST - 1; ++u) load(u, u);
@@ -321,14 +344,17 @@ __global__ void __launch_bounds__(NW * WAVE, WPS) k_gemm(GemmArgs a) {
             for (int t = 0; t < NT; ++t) {
                 ghalf8 wv;
                 __builtin_memcpy(&wv, &fw[0][t], 16);
+                f32x4_t part[MT];
 #pragma unroll
-                for (int p = 0; p < 2; ++p)
+                for (int p = 1; p >= 0; --p)
 #pragma unroll
                     for (int i = 0; i < MT; ++i) {
                         ghalf8 xv;
                         __builtin_memcpy(&xv, &fx[xs][i][p], 16);
-                        acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, xv, acc[i][t], 0, 0, 0);
+                        product(part[i], acc[i][t], wv, xv, p);
                     }
+#pragma unroll
+                for (int i = 0; i < MT; ++i) add(acc[i][t], part[i]);
                 if (more) load_w(0, t, s + 1);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -468,18 +494,18 @@ __global__ void __launch_bounds__(4 * WAVE, 2) k_attn_prompt(AttnArgs a) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) sc[h][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int st = 0; st < 4; ++st)
+        for (int p = 1; p >= 0; --p)                         // the small products first
 #pragma unroll
-            for (int p = 0; p < 2; ++p)
+            for (int st = 0; st < 4; ++st)
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
 #pragma unroll
                     for (int t = 0; t < 2; ++t)
                         sc[h][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[4 * t + st], qf[h][st][p], sc[h][t], 0, 0, 0);
         if (s + 4 < mine) load_k(s + 4);
-        ghalf8 ph[2], pl[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
+            ghalf8 ph, pl;
             float m = mx[h];
 #pragma unroll
             for (int t = 0; t < 2; ++t)
@@ -501,20 +527,18 @@ __global__ void __launch_bounds__(4 * WAVE, 2) k_attn_prompt(AttnArgs a) {
                     const float e = __builtin_amdgcn_exp2f((sc[h][t][r] - m) * a.scale);
                     ls += e;
                     const _Float16 hi = static_cast<_Float16>(e);
-                    ph[h][4 * t + r] = hi;
-                    pl[h][4 * t + r] = static_cast<_Float16>(e - static_cast<float>(hi));
+                    ph[4 * t + r] = hi;
+                    pl[4 * t + r] = static_cast<_Float16>(e - static_cast<float>(hi));
                 }
             sum[h] = sum[h] * corr + ls;
 #pragma unroll
-            for (int t = 0; t < 8; ++t) o[h][t] *= corr;
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
             for (int t = 0; t < 8; ++t) {
-                o[h][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t], ph[h], o[h][t], 0, 0, 0);
-                o[h][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t], pl[h], o[h][t], 0, 0, 0);
+                f32x4_t p = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t], pl, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                p = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t], ph, p, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[h][t][r] = fmaf(o[h][t][r], corr, p[r]);
             }
+        }
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -559,7 +583,9 @@ void launch_gemm(const GemmArgs &a, hipStream_t s) {
 // its own, so the tile is the smallest that still gives at most 256 blocks: a block's time is its
 // operand bytes (about 70 GB/s from L2 into one CU, whatever the other CUs do), and a block more
 // than CUs is a second round. Above 512 rows no tile gives that: there the one-slot form, two blocks to a
-// CU (768 rows: q|k|v 26 -> 23 us, gate|up 30 -> 23; 1001 rows 27.5 -> 26.5 and 30.5 -> 29).
+// CU (768 rows: gate|up 30 -> 25 us, with chained sums q|k|v 26 -> 23; its 32 x 128 tiles that add each step's
+// products 26.7), except q|k|v above 768 rows, whose 64 x 128 tiles do not fit half the registers with
+// a step's products beside the sums (1001 rows 32 us; chained in half the registers 26.5).
 void launch_qkv(const GemmArgs &a, hipStream_t s) {
     const int mt = (a.M + 15) / 16;
     if (mt <= 8) launch_gemm<1, 8, G_QKV, 4, 8, 2, 2>(a, s);
@@ -567,7 +593,7 @@ void launch_qkv(const GemmArgs &a, hipStream_t s) {
     else if (mt <= 24) launch_gemm<3, 8, G_QKV, 4, 8, 2, 1>(a, s);
     else if (mt <= 32) launch_gemm<4, 8, G_QKV, 4, 8, 2, 1>(a, s);
     else if (mt <= 48) launch_gemm<2, 8, G_QKV, 4, 8, 1, 2>(a, s);
-    else launch_gemm<4, 8, G_QKV, 4, 8, 1, 2, 2>(a, s);
+    else launch_gemm<4, 8, G_QKV, 4, 8, 2, 1>(a, s);
 }
 void launch_gate_up(const GemmArgs &a, hipStream_t s) {
     const int mt = (a.M + 15) / 16;
