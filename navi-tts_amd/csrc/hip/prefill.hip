@@ -18,9 +18,10 @@
 //  * The prefill's layers: five launches each. Up to 64 rows q|k|v, o, gate|up and down are whole-K
 //    row projections (rows.h) with the input RMSNorm, SwiGLU and the residual add fused in, and
 //    the attention (one block per row and kv group) applies the q/k head norms + RoPE and stores
-//    the f16 K/V row. Above, gemm.h's projections and attention, which hand every activation on as
-//    f16 pairs in MFMA fragment order. Either way the projections read the weights in the MFMA tile
-//    layout (rows.h pk_w), from a copy of every layer's weights tiled at create.
+//    the f16 K/V row. Above, gemm.h's projections, which add the same products in the same order, and an
+//    attention that reads the cache (up to 256 rows: the same bits again) or MFMA fragments. Either
+//    way the projections read the weights in the MFMA tile layout (rows.h pk_w), from a copy of
+//    every layer's weights tiled at create.
 #include "dev_common.h"
 #include "gemm.h"
 #include "host_util.h"
@@ -208,28 +209,36 @@ __global__ void __launch_bounds__(BT) k_swiglu(const float *part, int S, int M, 
     }
 }
 
-// Causal GQA attention of prompts of up to FUSED_ROWS rows from position 0 (above: gemm.h), one
-// block per (row m, kv group g) for its two q heads over keys 0..m (k_prefill_attention,
-// talker.hip:88-117), with the q/k head norms, RoPE and the f16 K/V store folded in (k_qk_norm_rope,
-// talker.hip:46-82). The block forms, from the raw q|k|v rows of the projection (`raw`, [rows][nq + 2
-// nkv heads] f32), its two q heads and the normed, rotated f16 keys and the f16 values 0..m of kv group
-// g in LDS, one wave per head row (lane l holding dims l and l + 64, the values 0 + x, so a -0 sum is
-// stored as +0), and stores K/V row m into the cache. Then wave w takes keys 64w .. 64w + 63; lane 16r
-// + c holds 16-byte chunk c of key 4i + r. Scores are summed over a key's 16 lanes by DPP; thread t
-// owns key t for the softmax; the score and value loops skip the groups of four keys past the row's.
+// Causal GQA attention of prompts of up to SHORT_KEYS rows from position 0 (above: gemm.h), one block per
+// (row m, kv group g) for its two q heads over keys 0..m (k_prefill_attention, talker.hip:88-117). Wave
+// w takes keys 64w .. 64w + 63; lane 16r + c holds 16-byte chunk c of key 4i + r. Scores are summed over
+// a key's 16 lanes by DPP; thread t owns key t for the softmax.
+// FUSED (up to FUSED_ROWS rows): the q/k head norms, RoPE and the f16 K/V store are folded in
+// (k_qk_norm_rope, talker.hip:46-82). The block forms, from the raw q|k|v rows of the projection (`raw`,
+// [rows][nq + 2 nkv heads] f32), its two q heads and the normed, rotated f16 keys and the f16 values
+// 0..m of kv group g in LDS, one wave per head row (lane l holding dims l and l + 64, the values 0 + x,
+// so a -0 sum is stored as +0), and stores K/V row m into the cache. Every key is in wave 0's range
+// then, so the score and value loops skip per group of four keys.
+// Otherwise the projection (gemm.h) has stored q and the cache rows: one load instruction covers four
+// whole 256-byte key rows, every K chunk goes out before the first score, the V chunks after the scores, so
+// they fly during the softmax and K and V never share the registers; the loops skip per wave (a per-group
+// exit measured slower). The output goes out in the o projection's layout: f32 tiles (rows.h pk_a)
+// when FUSED, f16 pairs (gemm.h pk_s) otherwise. The long prompts' matrix-core attention takes 16 rows
+// of a head at a time and would leave most of the chip idle here.
 constexpr int SHORT_KEYS = 256;
 constexpr int FUSED_ROWS = 64;
 struct HeadNorm {
     const float *raw, *qn, *kn, *invf;
     float eps;
 };
-__global__ void __launch_bounds__(BT) k_attn_prefill_short(uint16_t *kc, uint16_t *vc, int nq, int nkv, float scale, float *out,
-                                                           int ldo, HeadNorm hn) {
+template <bool FUSED>
+__global__ void __launch_bounds__(BT) k_attn_prefill_short(const float *q, uint16_t *kc, uint16_t *vc, int nq, int nkv, float scale,
+                                                           float *out, int ldo, uint32_t *flag, HeadNorm hn) {
     constexpr int NWV = BT / WAVE, KW = SHORT_KEYS / NWV, KI = KW / 4;
     static_assert(SHORT_KEYS == BT, "one key per thread in the softmax");
-    static_assert(FUSED_ROWS <= KW, "every key in wave 0's range");
+    static_assert(FUSED_ROWS <= KW, "fused: every key in wave 0's range");
     __shared__ float qs[2][HD], sc[2][SHORT_KEYS], red[2][NWV], opart[NWV][4][2][HD];
-    __shared__ uint16_t ks[FUSED_ROWS][HD], vs[FUSED_ROWS][HD];
+    __shared__ uint16_t ks[FUSED ? FUSED_ROWS : 1][HD], vs[FUSED ? FUSED_ROWS : 1][HD];
     // grid (kv groups, rows): blocks go out in row order from the last row (the most keys) down,
     // every kv group of a row together, so the blocks that wait for a free slot are the shortest;
     // and kv group g's blocks all land on XCD g (block id % 8), whose L2 then holds its keys
@@ -237,51 +246,62 @@ __global__ void __launch_bounds__(BT) k_attn_prefill_short(uint16_t *kc, uint16_
     const int QD = nq * HD, KVD = nkv * HD;
     const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, r = l >> 4;
     u32x4_t kr[KI], vr[KI];
-    // task t: q head 2g + t of row m (t < 2), else key / value row j = t - 2 of kv group g
-    const int W = QD + 2 * KVD;
-    for (int t = wv; t < 2 + n; t += NWV) {
-        const bool isq = t < 2;
-        const int row = isq ? m : t - 2;
-        const float *hp = hn.raw + static_cast<size_t>(row) * W + (isq ? (2 * g + t) * HD : QD + g * HD);
-        const float *vp = hn.raw + static_cast<size_t>(row) * W + QD + KVD + g * HD;
-        const float a0 = 0.f + gld(hp + l), a1 = 0.f + gld(hp + l + HD / 2);
-        float b0 = 0.f, b1 = 0.f;
-        if (!isq) {
-            b0 = 0.f + gld(vp + l);
-            b1 = 0.f + gld(vp + l + HD / 2);
-        }
-        float sn, cs;
-        sincosf(static_cast<float>(row) * gld(hn.invf + l), &sn, &cs);
-        const float *nw = isq ? hn.qn : hn.kn;
-        const float scl = rsqrtf(wave_sum(fmaf(a0, a0, a1 * a1)) / static_cast<float>(HD) + hn.eps);
-        const float x0 = a0 * scl * gld(nw + l), x1 = a1 * scl * gld(nw + l + HD / 2);
-        const float y0 = x0 * cs - x1 * sn;
-        const float y1 = x1 * cs + x0 * sn;
-        if (isq) {
-            qs[t][l] = y0;
-            qs[t][l + HD / 2] = y1;
-        } else {
-            const uint16_t k0 = f2h(y0), k1 = f2h(y1), v0 = f2h(b0), v1 = f2h(b1);
-            ks[row][l] = k0;
-            ks[row][l + HD / 2] = k1;
-            vs[row][l] = v0;
-            vs[row][l + HD / 2] = v1;
-            if (row == m) {
-                uint16_t *kd = kc + static_cast<size_t>(m) * KVD + g * HD, *vd = vc + static_cast<size_t>(m) * KVD + g * HD;
-                gst(kd + l, k0);
-                gst(kd + l + HD / 2, k1);
-                gst(vd + l, v0);
-                gst(vd + l + HD / 2, v1);
+    if constexpr (FUSED) {
+        // task t: q head 2g + t of row m (t < 2), else key / value row j = t - 2 of kv group g
+        const int W = QD + 2 * KVD;
+        for (int t = wv; t < 2 + n; t += NWV) {
+            const bool isq = t < 2;
+            const int row = isq ? m : t - 2;
+            const float *hp = hn.raw + static_cast<size_t>(row) * W + (isq ? (2 * g + t) * HD : QD + g * HD);
+            const float *vp = hn.raw + static_cast<size_t>(row) * W + QD + KVD + g * HD;
+            const float a0 = 0.f + gld(hp + l), a1 = 0.f + gld(hp + l + HD / 2);
+            float b0 = 0.f, b1 = 0.f;
+            if (!isq) {
+                b0 = 0.f + gld(vp + l);
+                b1 = 0.f + gld(vp + l + HD / 2);
+            }
+            float sn, cs;
+            sincosf(static_cast<float>(row) * gld(hn.invf + l), &sn, &cs);
+            const float *nw = isq ? hn.qn : hn.kn;
+            const float scl = rsqrtf(wave_sum(fmaf(a0, a0, a1 * a1)) / static_cast<float>(HD) + hn.eps);
+            const float x0 = a0 * scl * gld(nw + l), x1 = a1 * scl * gld(nw + l + HD / 2);
+            const float y0 = x0 * cs - x1 * sn;
+            const float y1 = x1 * cs + x0 * sn;
+            if (isq) {
+                qs[t][l] = y0;
+                qs[t][l + HD / 2] = y1;
+            } else {
+                const uint16_t k0 = f2h(y0), k1 = f2h(y1), v0 = f2h(b0), v1 = f2h(b1);
+                ks[row][l] = k0;
+                ks[row][l + HD / 2] = k1;
+                vs[row][l] = v0;
+                vs[row][l + HD / 2] = v1;
+                if (row == m) {
+                    uint16_t *kd = kc + static_cast<size_t>(m) * KVD + g * HD, *vd = vc + static_cast<size_t>(m) * KVD + g * HD;
+                    gst(kd + l, k0);
+                    gst(kd + l + HD / 2, k1);
+                    gst(vd + l, v0);
+                    gst(vd + l + HD / 2, v1);
+                }
             }
         }
-    }
-    __syncthreads();                                  // qs, ks, vs
+        __syncthreads();                                  // qs, ks, vs
 #pragma unroll
-    for (int i = 0; i < KI; ++i) {
-        const int j = wv * KW + 4 * i + r;
-        kr[i] = j < n ? *reinterpret_cast<const u32x4_t *>(&ks[j][c * 8]) : u32x4_t{0u, 0u, 0u, 0u};
-        vr[i] = j < n ? *reinterpret_cast<const u32x4_t *>(&vs[j][c * 8]) : u32x4_t{0u, 0u, 0u, 0u};
+        for (int i = 0; i < KI; ++i) {
+            const int j = wv * KW + 4 * i + r;
+            kr[i] = j < n ? *reinterpret_cast<const u32x4_t *>(&ks[j][c * 8]) : u32x4_t{0u, 0u, 0u, 0u};
+            vr[i] = j < n ? *reinterpret_cast<const u32x4_t *>(&vs[j][c * 8]) : u32x4_t{0u, 0u, 0u, 0u};
+        }
+    } else {
+        qs[threadIdx.x >> 7][threadIdx.x & (HD - 1)] = gld(q + static_cast<size_t>(m) * QD + g * 2 * HD + threadIdx.x);
+        const uint16_t *kb = kc + g * HD + c * 8;
+#pragma unroll
+        for (int i = 0; i < KI; ++i) {
+            const int j = wv * KW + 4 * i + r;
+            kr[i] = j < n ? *(const NAVI_GLOBAL u32x4_t *) (kb + static_cast<size_t>(j) * KVD) : u32x4_t{0u, 0u, 0u, 0u};
+        }
     }
+    __syncthreads();                                      // qs
     {
         float q0[8], q1[8];
 #pragma unroll
@@ -291,7 +311,7 @@ __global__ void __launch_bounds__(BT) k_attn_prefill_short(uint16_t *kc, uint16_
         }
 #pragma unroll
         for (int i = 0; i < KI; ++i) {
-            if (wv * KW + 4 * i >= n) break;  // this wave's remaining keys are past the row's
+            if (wv * KW + (FUSED ? 4 * i : 0) >= n) break;  // this wave's remaining keys are past the row's
             uint4 k4;
             __builtin_memcpy(&k4, &kr[i], 16);
             float a0 = dot8(k4, q0, 0.f), a1 = dot8(k4, q1, 0.f);
@@ -308,6 +328,17 @@ __global__ void __launch_bounds__(BT) k_attn_prefill_short(uint16_t *kc, uint16_
                 sc[0][j] = a0 * scale;
                 sc[1][j] = a1 * scale;
             }
+        }
+    }
+    if constexpr (!FUSED) {
+        // prompts of 65-256 rows: the V chunks go out after the scores and fly during the softmax,
+        // so K and V are never in registers together (about 100 VGPRs instead of 156: four blocks
+        // per CU instead of three; the sums are unchanged)
+        const uint16_t *vb = vc + g * HD + c * 8;
+#pragma unroll
+        for (int i = 0; i < KI; ++i) {
+            const int j = wv * KW + 4 * i + r;
+            vr[i] = j < n ? *(const NAVI_GLOBAL u32x4_t *) (vb + static_cast<size_t>(j) * KVD) : u32x4_t{0u, 0u, 0u, 0u};
         }
     }
     __syncthreads();
@@ -330,7 +361,7 @@ __global__ void __launch_bounds__(BT) k_attn_prefill_short(uint16_t *kc, uint16_
         for (int e = 0; e < 8; ++e) o0[e] = o1[e] = 0.f;
 #pragma unroll
         for (int i = 0; i < KI; ++i) {
-            if (wv * KW + 4 * i >= n) break;  // zero weights (and zero rows) from here on
+            if (wv * KW + (FUSED ? 4 * i : 0) >= n) break;  // zero weights (and zero rows) from here on
             const int j = wv * KW + 4 * i + r;
             const float p0 = sc[0][j], p1 = sc[1][j];
             half8_t hv;
@@ -356,7 +387,13 @@ __global__ void __launch_bounds__(BT) k_attn_prefill_short(uint16_t *kc, uint16_
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) acc += opart[w][rr][hh][d];
     const float sum = red[hh][0] + red[hh][1] + red[hh][2] + red[hh][3];
-    gst(out + rows::pk_a(m, (g * 2 + hh) * HD + d, ldo), acc / sum);
+    if constexpr (FUSED) {
+        gst(out + rows::pk_a(m, (g * 2 + hh) * HD + d, ldo), acc / sum);
+    } else {
+        bool bad = false;
+        gm::split_store(reinterpret_cast<uint16_t *>(out) + gm::pk_s(m, (g * 2 + hh) * HD + d, ldo), acc / sum, bad);
+        if (bad) gst(flag, 1u);
+    }
 }
 
 // rows[t] = table[ids[t]] (f16 -> f32), k_gather_rows (talker.hip:20-25).
@@ -519,10 +556,10 @@ struct navi_talker {
     // work buffers
     // x (the residual stream), att and h in the tile layout (rows.h pk_a), the rest row-major
     float *x = nullptr, *xn = nullptr, *q = nullptr, *att = nullptr, *h = nullptr, *part = nullptr, *invf = nullptr;
-    // prompts above FUSED_ROWS rows (gemm.h): the normed residual rows as f16 pairs, their partial sums
-    // of squares, the rotation of every position and the prompt's keys and values as MFMA fragments
-    uint16_t *xs = nullptr, *kf = nullptr, *vf = nullptr;
-    float *ssq = nullptr, *rot = nullptr;
+    // prompts above FUSED_ROWS rows (gemm.h): the rotation of every position and, above SHORT_KEYS, the
+    // prompt's keys and values as MFMA fragments; att and h hold f16 pairs (gemm.h pk_s) there, q too above SHORT_KEYS
+    uint16_t *kf = nullptr, *vf = nullptr;
+    float *rot = nullptr;
     size_t part_floats = 0;
     uint32_t *flag = nullptr;
     bool flag_set = false;             // whether a call may have left the flag set
@@ -699,10 +736,8 @@ navi_status navi_talker_create(const navi_model_params *p, const navi_tensor_ref
     TALLOC(t->x, MT16 * t->H);
     TALLOC(t->xn, M * t->H);
     TALLOC(t->q, MT16 * t->QD);
-    TALLOC(t->xs, 2 * MT16 * t->H);
     TALLOC(t->kf, (M + 31) / 32 * 32 * t->KVD);
     TALLOC(t->vf, (M + 31) / 32 * 32 * t->KVD);
-    TALLOC(t->ssq, gm::SSQ * M);
     TALLOC(t->rot, M * HD);
     TALLOC(t->att, MT16 * t->QD);
     TALLOC(t->h, MT16 * t->F);
@@ -874,9 +909,9 @@ namespace {
 // last row's final RMSNorm (the post-norm hidden the frame takes) and the codec head. Up to FUSED_ROWS
 // rows: q|k|v with the RMSNorm fused -> attention with the q/k norms, RoPE and the K/V store -> o (+
 // residual) -> gate|up with the RMSNorm and SwiGLU fused -> down (+ residual), every projection one
-// whole-K MFMA kernel on the tiled operands (rows.h). Above: gemm.h's kernels, every activation
-// handed on as f16 pairs in fragment order (t.xs and t.ssq from k_split_rows). false: a projection
-// shape the tiled kernels do not take (nothing after it was launched).
+// whole-K MFMA kernel on the tiled operands (rows.h). Above: gemm.h's projections, the attention's and
+// the MLP's outputs handed on as f16 pairs in fragment order. false: a projection shape the tiled
+// kernels do not take (nothing after it was launched).
 bool prefill_layers(navi_talker &t, int T, hipStream_t s) {
     const int H = t.H, QKVW = t.QD + 2 * t.KVD;
     const float scale = 1.f / std::sqrt(static_cast<float>(HD));
@@ -884,61 +919,65 @@ bool prefill_layers(navi_talker &t, int T, hipStream_t s) {
         const LayerW &w = t.layers[l];
         if (T > FUSED_ROWS) {
             auto half = [](float *p) { return reinterpret_cast<uint16_t *>(p); };
+            const bool wide = T > SHORT_KEYS;
             gm::GemmArgs a{};
             a.flag = t.flag;
             a.M = T;
             a.eps = t.eps;
-            a.ssq_in = a.ssq_out = t.ssq;
-            a.ldq = t.mmax;
             gm::GemmArgs b = a;
-            b.x = t.xs;
+            b.x = t.x;
             b.w = w.qkv_t;
             b.K = H;
             b.N = QKVW;
+            b.ln = w.ln1;
             b.qn = w.qn;
             b.kn = w.kn;
             b.cs = t.rot;
-            b.q = half(t.q);
+            b.qf = wide ? nullptr : t.q;
+            b.qs = half(t.q);
             b.kc = t.kk[l];
             b.vc = t.vv[l];
-            b.kf = t.kf;
-            b.vf = t.vf;
+            b.kf = wide ? t.kf : nullptr;
+            b.vf = wide ? t.vf : nullptr;
             b.q_scale = w.q_scale;
             b.nq = t.NQ;
             b.nkv = t.NKV;
             gm::launch_qkv(b, s);
-            hipLaunchKernelGGL(gm::k_attn_prompt, dim3(t.NKV, (T + 15) / 16), dim3(4 * WAVE), 0, s,
-                               gm::AttnArgs{half(t.q), t.kf, t.vf, half(t.att), t.flag, T, t.NQ, static_cast<float>(1.4426950408889634 / (std::sqrt(static_cast<double>(HD)) * w.q_scale))});
+            if (wide)
+                hipLaunchKernelGGL(gm::k_attn_prompt, dim3(t.NQ, (T + 15) / 16), dim3(4 * WAVE), 0, s,
+                                   gm::AttnArgs{half(t.q), t.kf, t.vf, half(t.att), t.flag, T, t.NQ, scale / w.q_scale});
+            else
+                hipLaunchKernelGGL(k_attn_prefill_short<false>, dim3(t.NKV, T), dim3(BT), 0, s, t.q, t.kk[l], t.vv[l], t.NQ, t.NKV,
+                                   scale, t.att, t.QD, t.flag, HeadNorm{});
             b = a;
-            b.x = half(t.att);
+            b.x = t.att;
             b.w = w.o_t;
             b.K = t.QD;
             b.N = H;
             b.res = t.x;
             b.ln = w.ln2;
-            b.y = t.xs;
-            gm::launch_resid<64>(b, s);
+            gm::launch_resid<4>(b, s);
             b = a;
-            b.x = t.xs;
+            b.x = t.x;
             b.w = w.gu_t;
             b.K = H;
             b.N = t.F;
+            b.ln = w.ln2;
             b.y = half(t.h);
             gm::launch_gate_up(b, s);
             b = a;
-            b.x = half(t.h);
+            b.x = t.h;
             b.w = w.d_t;
             b.K = t.F;
             b.N = H;
             b.res = t.x;
             b.ln = l + 1 < t.L ? t.layers[l + 1].ln1 : nullptr;
-            b.y = t.xs;
-            gm::launch_resid<96>(b, s);
+            gm::launch_resid<6>(b, s);
             continue;
         }
         if (!rows::launch_rows_pk(rows::EPI_PLAIN, true, t.x, T, H, w.ln1, t.eps, w.qkv_t, QKVW, t.part, QKVW, t.flag, s)) return false;
-        hipLaunchKernelGGL(k_attn_prefill_short, dim3(t.NKV, T), dim3(BT), 0, s, t.kk[l], t.vv[l], t.NQ, t.NKV, scale, t.att, t.QD,
-                           HeadNorm{t.part, w.qn, w.kn, t.invf, t.eps});
+        hipLaunchKernelGGL(k_attn_prefill_short<true>, dim3(t.NKV, T), dim3(BT), 0, s, nullptr, t.kk[l], t.vv[l], t.NQ, t.NKV, scale, t.att,
+                           t.QD, t.flag, HeadNorm{t.part, w.qn, w.kn, t.invf, t.eps});
         if (!rows::launch_rows_pk(rows::EPI_RESID, false, t.att, T, t.QD, nullptr, 0.f, w.o_t, H, t.x, 0, t.flag, s) ||
             !rows::launch_rows_pk(rows::EPI_SWIGLU, true, t.x, T, H, w.ln2, t.eps, w.gu_t, t.F, t.h, 0, t.flag, s) ||
             !rows::launch_rows_pk(rows::EPI_RESID, false, t.h, T, t.F, nullptr, 0.f, w.d_t, H, t.x, 0, t.flag, s))
@@ -971,7 +1010,7 @@ navi_status navi_talker_prefill(navi_talker *t, const float *d_rows, int32_t n_r
     // the rows into the layers' layout; the f16-range flag is clear when the layers start
     if (T > FUSED_ROWS) {
         if (t->flag_set) NAVI_TRY_HIP(hipMemsetAsync(t->flag, 0, 4, s), err, errlen);
-        hipLaunchKernelGGL(gm::k_split_rows, dim3(T), dim3(256), 0, s, d_rows, t->layers[0].ln1, t->x, t->xs, t->ssq, t->mmax, t->flag);
+        hipLaunchKernelGGL(gm::k_rows_in, dim3(T), dim3(256), 0, s, d_rows, t->layers[0].ln1, t->x, t->flag);
     } else {
         rows::tile_rows(d_rows, T, H, t->x, s, t->flag);
     }
