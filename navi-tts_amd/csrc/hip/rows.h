@@ -336,9 +336,10 @@ void launch_pk(int M, int N, const RowArgs &ra, hipStream_t s) {
 // 4 (gate|up, o) or 2 (down) column groups per block; up to 64 rows the one-group kernels, except
 // q|k|v at 17-32 rows, where two groups halve the reads of the second row tile. o and down have 64 column
 // tiles, a quarter of the CUs: up to 16 rows four blocks share each (a 10-row prompt 1.07 -> 1.03 ms),
-// up to 64 two blocks share each row tile (in place of two that share the columns and all read the rows,
-// with q|k|v's two groups: 32 streams 4.51 -> 4.43 ms a step). Every
-// shape keeps the row-major kernels' split of K over the waves, so the outputs are theirs bit for
+// up to 32 two blocks share each row tile (in place of two that share the columns and all read the rows,
+// with q|k|v's two groups: 32 streams 4.51 -> 4.43 ms a step); above, one block per tile already gives 192 of
+// the 256 CUs, and a block fills one, so twice as many take two rounds (prompts of 33, 48 and 64 rows
+// 1.28, 1.41 and 1.55 ms, shared 1.41, 1.53 and 1.69). Every shape keeps the row-major kernels' split of K over the waves, so the outputs are theirs bit for
 // bit (gate|up over 16 waves x 2 steps measured 0.7 us faster at 130 rows, with other bits).
 // false: a shape these kernels do not take.
 bool launch_rows_pk(int epi, bool norm, const float *A, int M, int K, const float *ln, float eps, const uint16_t *w, int N,
@@ -368,13 +369,15 @@ bool launch_rows_pk(int epi, bool norm, const float *A, int M, int K, const floa
         if (wide && M <= 96) launch_pk<1, EPI_RESID, false, 16, 4, 2>(M, N, ra, s);   // more blocks where they are few
         else if (wide) launch_pk<1, EPI_RESID, false, 16, 4, 4>(M, N, ra, s);
         else if (M <= 16) launch_pk<1, EPI_RESID, false, 16, 4, 1, 4>(M, N, ra, s);
-        else launch_pk<1, EPI_RESID, false, 16, 4, 1, 1, 2>(M, N, ra, s);
+        else if (M <= 32) launch_pk<1, EPI_RESID, false, 16, 4, 1, 1, 2>(M, N, ra, s);
+        else launch_pk<1, EPI_RESID, false, 16, 4, 1>(M, N, ra, s);
         return true;
     }
     if (epi == EPI_RESID && K == 3072) {
         if (wide) launch_pk<1, EPI_RESID, false, 16, 6, 2>(M, N, ra, s);
         else if (M <= 16) launch_pk<1, EPI_RESID, false, 16, 6, 1, 4>(M, N, ra, s);
-        else launch_pk<1, EPI_RESID, false, 16, 6, 1, 1, 2>(M, N, ra, s);
+        else if (M <= 32) launch_pk<1, EPI_RESID, false, 16, 6, 1, 1, 2>(M, N, ra, s);
+        else launch_pk<1, EPI_RESID, false, 16, 6, 1>(M, N, ra, s);
         return true;
     }
     return false;

@@ -1,10 +1,12 @@
 """A row's results do not depend on how many rows a prompt has: every projection adds the same products in
 the same order at every row count, so the rows of a longer prompt are a shorter one's bit for bit.
 
-Up to 256 rows the reference is the 64-row prompt, the most the whole-K row kernels take (rows.h): above
-it the streamed projections (gemm.h) and the attention that reads the cache have to give its bits. Above 256
-rows the attention is the matrix cores' in 256-key chunks, with bits of its own from the second layer on:
-the reference is the 257-row prompt there, and the 64-row one for the first layer's keys and values.
+Up to 64 rows the whole-K row kernels share their tiles between blocks by the row count (rows.h): the
+reference is the 10-row prompt. From there to 256 rows it is the 64-row prompt, the most those kernels
+take: above it the streamed projections (gemm.h) and the attention that reads the cache have to give its
+bits. Above 256 rows the attention is the matrix cores' in 256-key chunks, with bits of its own from the
+second layer on: the reference is the 257-row prompt there, and the 64-row one for the first layer's
+keys and values.
 """
 import numpy as np
 import pytest
@@ -29,7 +31,7 @@ def side(small_blob):
     def prefill(T):
         t.prefill(d.ptr, T)
         return [t.kv.read(l, T) for l in range(ora.tp.n_layer)]
-    yield prefill, t, ora, rows, {n: prefill(n) for n in (64, 257)}
+    yield prefill, t, ora, rows, {n: prefill(n) for n in (10, 64, 257)}
     t.close()
 
 
@@ -37,6 +39,12 @@ def _same(got, want, layers, n):
     for l in layers:
         for a, b in zip(got[l], want[l]):
             np.testing.assert_array_equal(a[:n], b[:n])
+
+
+@pytest.mark.parametrize("T", [16, 17, 32, 33, 48, 49, 64])
+def test_shared_tiles_have_the_same_bits(side, T):
+    prefill, _, ora, _, want = side
+    _same(prefill(T), want[10], range(ora.tp.n_layer), 10)
 
 
 # every tile choice of the streamed projections (gemm.h's launch rules), its first and last row counts
