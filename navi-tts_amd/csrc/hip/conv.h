@@ -6,6 +6,7 @@
 #pragma once
 
 #include "dev_common.h"
+#include "snake.h"
 
 namespace navi_amd {
 namespace cv {
@@ -54,65 +55,6 @@ struct ConvArgs {
 };
 
 __device__ __forceinline__ float silu(float g) { return g / (1.f + expf(-g)); }
-
-// sin^2(u). Its period is pi and it is even, so no quadrant has to be told apart: r = u - n pi, |r| <= pi /
-// 2 (pi as two floats; the first product is exact and so is its difference from u), then a polynomial
-// in z = r^2, z + z^2 P(z) with P fitted to (sin^2(sqrt z) - z) / z^2 (least squares on Chebyshev nodes,
-// reweighted towards the smallest maximum: 2e-10 over |r| <= 1.64). 13 instructions where sinf(u)^2 takes
-// about three times as many and a branch to its reduction for large arguments at every use: the
-// epilogues' sines took longer than their MFMAs (last decoder block's residual unit at 240 frames 394
-// -> 289 us, a 240-frame block 5.50 -> 4.84 ms, 52 streamed frames 3.69 -> 3.45). Root mean square
-// error 3.4e-8 for |u| up to 2^20 (a correctly rounded sinf squared: 2.7e-8); the PCM's distance from 64
-// bits stays 1.2e-6. Larger arguments, which no activation inside the f16 range gives with a sane
-// alpha, reduce in double.
-constexpr float SIN2_MAX = 1048576.f;
-__device__ __forceinline__ float sin2_poly(float r) {
-    const float z = r * r;
-    float p = fmaf(7.925196854330352e-8f, z, -4.2174178815912455e-6f);
-    p = fmaf(p, z, 1.40975636895746e-4f);
-    p = fmaf(p, z, -3.174476558342576e-3f);
-    p = fmaf(p, z, 4.444437846541405e-2f);
-    p = fmaf(p, z, -3.333333134651184e-1f);
-    return fmaf(z * z, p, z);
-}
-__device__ __forceinline__ float sin2_reduce(float u) {
-    const float n = rintf(u * 0.318309873f);
-    return fmaf(-n, -8.74227766e-8f, fmaf(-n, 3.14159274f, u));
-}
-// A pass leaves less than 2^-51 of an argument whose multiple of pi has more than 53 bits (2.8e16 on): three
-// bring every finite float into the polynomial's range. The phase holds up to about 2^80.
-__device__ __forceinline__ float sin2_reduce_wide(float u) {
-    double r = static_cast<double>(u);
-#pragma unroll 1
-    for (int pass = 0; pass < 3; ++pass) {
-        const double m = rint(r * 0.3183098861837907);
-        r = fma(-m, 1.2246467991473532e-16, fma(-m, 3.141592653589793, r));
-    }
-    return static_cast<float>(r);
-}
-
-// v + zb sin^2(za v) for N values of one channel: one branch for all of them, their chains interleaved.
-template <int N>
-__device__ __forceinline__ void snake_n(const float (&v)[N], float za, float zb, float (&out)[N]) {
-    float big = 0.f;
-#pragma unroll
-    for (int i = 0; i < N; ++i) big = fmaxf(big, fabsf(v[i] * za));
-#pragma unroll
-    for (int i = 0; i < N; ++i) out[i] = sin2_reduce(v[i] * za);
-    if (__builtin_expect(big > SIN2_MAX, 0)) {
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-            if (fabsf(v[i] * za) > SIN2_MAX) out[i] = sin2_reduce_wide(v[i] * za);
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) out[i] = fmaf(sin2_poly(out[i]), zb, v[i]);
-}
-__device__ __forceinline__ float snake(float v, float za, float zb) {
-    const float a[1] = {v};
-    float o[1];
-    snake_n(a, za, zb, o);
-    return o[0];
-}
 
 // The per-output-channel operands of the epilogue, loaded once per thread (a thread's outputs
 // share their channel).
