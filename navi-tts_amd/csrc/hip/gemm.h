@@ -18,9 +18,9 @@
 //
 // What bounds them: the operand bytes into a CU (about 70 GB/s from L2), then the exchange and the waits of
 // the end. Against the row kernels (16-row blocks, which read every weight once per 16 rows): a prefill of
-// 65 rows 1.23 -> 1.06 ms, 130 1.85 -> 1.33, 300 3.02 -> 1.63, 1001 9.23 -> 3.88.
-// Fewer, longer runs or sums that start from zero at every step save an exchange (1001 rows 3.28 ms), but give
-// other bits: K/V rows are then up to 12 % further from 64 bits in the layers between the first and the last,
+// 65 rows 1.22 -> 1.06 ms, 130 1.85 -> 1.34, 300 3.01 -> 1.64, 768 6.66 -> 3.26, 1001 9.24 -> 3.92.
+// Four waves of longer runs, whose sums start from zero at every step, exchange half as much (256 rows 1.44
+// ms instead of 1.66, with the attention on the matrix cores; 768 2.80, 1001 3.32), but give other bits: K/V rows are then up to 12 % further from 64 bits in the layers between the first and the last,
 // and a row's results depend on the length of its prompt.
 #pragma once
 
@@ -559,24 +559,36 @@ void launch_gemm(const GemmArgs &a, hipStream_t s) {
 
 // The talker's shapes (K 1024 into q|k|v and gate|up, 2048 into o, 3072 into down; N 4096, 2 x 3072,
 // 1024, 1024). A block's time is its operand bytes (about 70 GB/s from L2 into one CU, whatever the other
-// CUs do), and a block more than CUs is a second round, so the tile is the smallest that still gives at most
-// 256 blocks, up to the largest whose sums fit the registers of eight waves (64 x 128).
+// CUs do) and its end, a block fills a CU, and a block more than CUs is a second round: the tile is the one
+// whose rounds take least.
+int rounds(int ncol, int mtiles, int MT) { return (ncol * ((mtiles + MT - 1) / MT) + 255) / 256; }
+
+// 16 MT x 128 tiles take 6.6, 9, 12.3 and 15.3 us a round for MT = 1 .. 4, as MT + 1. 640 rows: two rounds of
+// MT = 3 23.6 us, three of MT = 2 25.1, two of MT = 4 27.9; 1001: two of MT = 4 30.8, three of MT = 3 36.3.
 void launch_qkv(const GemmArgs &a, hipStream_t s) {
-    const int mt = (a.M + 15) / 16;
-    if (mt <= 8) launch_gemm<1, 8, G_QKV, 8, 1, 4, 4, 2, 1>(a, s);
-    else if (mt <= 16) launch_gemm<2, 8, G_QKV, 8, 1, 4, 2, 2, 1>(a, s);
-    else if (mt <= 24) launch_gemm<3, 8, G_QKV, 8, 1, 4, 1, 2, 1>(a, s);
+    const int mt = (a.M + 15) / 16, ncol = a.N / 128;
+    int best = 1;
+    for (int MT = 2; MT <= 4; ++MT)
+        if (rounds(ncol, mt, MT) * (MT + 1) < rounds(ncol, mt, best) * (best + 1)) best = MT;
+    if (best == 1) launch_gemm<1, 8, G_QKV, 8, 1, 4, 4, 2, 1>(a, s);
+    else if (best == 2) launch_gemm<2, 8, G_QKV, 8, 1, 4, 1, 2, 1>(a, s);
+    else if (best == 3) launch_gemm<3, 8, G_QKV, 8, 1, 4, 1, 2, 1>(a, s);
     else launch_gemm<4, 8, G_QKV, 8, 1, 4, 1, 2, 1>(a, s);
 }
+// One round: 16 x 128 tiles up to 5 row tiles (7.7 us), 32 x 96 up to 8 (8.4; 16 x 128 would be a second round, 12.3),
+// 32 x 128 up to 10 (9.1). Above, 32 x 192 tiles (12.2 us a round of 256 rows) or 64 x 128 (13.5 a round of 340),
+// whichever takes fewer rounds: 320 rows 19.6 and 13.6 us, 512 22.5 and 24.7, 640 30.5 and 25.2, 1001 47.5 and 38.0.
 void launch_gate_up(const GemmArgs &a, hipStream_t s) {
     const int mt = (a.M + 15) / 16;
     if (mt <= 5) launch_gemm<1, 8, G_SWIGLU, 8, 1, 4, 4, 2, 1>(a, s);
     else if (mt <= 8) launch_gemm<2, 6, G_SWIGLU, 8, 1, 4, 2, 2, 2>(a, s);
     else if (mt <= 10) launch_gemm<2, 8, G_SWIGLU, 8, 1, 4, 2, 2, 2>(a, s);
-    else if (mt <= 16) launch_gemm<4, 6, G_SWIGLU, 8, 1, 4, 1, 2, 2>(a, s);
+    else if (rounds(a.N / 96, mt, 2) <= rounds(a.N / 64, mt, 4)) launch_gemm<2, 12, G_SWIGLU, 8, 1, 4, 1, 2, 1>(a, s);
     else launch_gemm<4, 8, G_SWIGLU, 8, 1, 4, 1, 2, 2>(a, s);
 }
-// PER = K / 512
+// PER = K / 512. The smallest tile that gives at most one round, up to 64 x 64. Down at 128 rows: 16 x 32 tiles 5.8
+// us, 32 x 32 7.3; 256: 32 x 32 7.6, 32 x 64 9.3, 16 x 32 in two rounds 9.6; 512: 32 x 64 11.9, 64 x 64 16.4; 513:
+// 16.5 in one round of 64 x 64, 18.9 in two of 32 x 64; 1001: 20.0 and 31.2.
 template <int PER>
 void launch_resid(const GemmArgs &a, hipStream_t s) {
     const int mt = (a.M + 15) / 16;

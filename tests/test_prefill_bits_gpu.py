@@ -48,13 +48,13 @@ def test_shared_tiles_have_the_same_bits(side, T):
 
 
 # every tile choice of the streamed projections (gemm.h's launch rules), its first and last row counts
-@pytest.mark.parametrize("T", [65, 80, 81, 128, 129, 160, 161, 200, 256])
+@pytest.mark.parametrize("T", [65, 80, 81, 128, 129, 160, 161, 200, 240, 256])
 def test_rows_have_the_row_kernels_bits(side, T):
     prefill, _, ora, _, want = side
     _same(prefill(T), want[64], range(ora.tp.n_layer), 64)
 
 
-@pytest.mark.parametrize("T", [300, 320, 321, 384, 385, 512, 513, 768, 769, 1001, 1025, 2056])
+@pytest.mark.parametrize("T", [300, 320, 321, 384, 385, 512, 513, 640, 641, 768, 769, 1001, 1025, 2056])
 def test_long_prompts_rows_are_the_shorter_ones(side, T):
     prefill, _, ora, _, want = side
     got = prefill(T)
