@@ -174,41 +174,6 @@ __global__ void __launch_bounds__(BT) k_finish_linear(const float *part, int S, 
     }
 }
 
-// x[m] = (S > 0 ? sum_s part + x[m] : src[m]); xn[m] = RMSNorm(x[m]) * w (k_rmsnorm, kernels.h:342-350,
-// fused with the residual epilogue of the o / down projections).
-__global__ void __launch_bounds__(BT) k_resid_norm(const float *part, int S, const float *src, float *x, const float *w,
-                                                   float eps, float *xn, int M, int H) {
-    __shared__ float red[4];
-    const int m = blockIdx.x, i = threadIdx.x * 4;            // H == 4 * BT
-    const size_t idx = static_cast<size_t>(m) * H + i;
-    const f32x4_t v = S > 0 ? sum_parts4(part, S, static_cast<size_t>(M) * H, idx) + ld4(x + idx) : ld4(src + idx);
-    const f32x4_t wv = ld4(w + i);
-    st4(x + idx, v);
-    float ss = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) ss = fmaf(v[j], v[j], ss);
-    ss = block_sum256(ss, red);
-    const float scale = rsqrtf(ss / static_cast<float>(H) + eps);
-    f32x4_t o;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = v[j] * scale * wv[j];
-    st4(xn + idx, o);
-}
-
-// h[m][c] = SiLU(gate) * up from the [gate | up] partials (PRO_SILU_GATE / k_silu_gate, kernels.h:334-340).
-__global__ void __launch_bounds__(BT) k_swiglu(const float *part, int S, int M, int F, float *h) {
-    const int m = blockIdx.x;
-    const size_t stride = static_cast<size_t>(M) * 2 * F;
-    for (int c = threadIdx.x * 4; c < F; c += BT * 4) {
-        const f32x4_t g = sum_parts4(part, S, stride, static_cast<size_t>(m) * 2 * F + c);
-        const f32x4_t u = sum_parts4(part, S, stride, static_cast<size_t>(m) * 2 * F + F + c);
-        f32x4_t o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = silu(g[j]) * u[j];
-        st4(h + static_cast<size_t>(m) * F + c, o);
-    }
-}
-
 // Causal GQA attention of prompts of up to SHORT_KEYS rows from position 0 (above: gemm.h), one block per
 // (row m, kv group g) for its two q heads over keys 0..m (k_prefill_attention, talker.hip:88-117). Wave
 // w takes keys 64w .. 64w + 63; lane 16r + c holds 16-byte chunk c of key 4i + r. Scores are summed over
@@ -456,20 +421,6 @@ void launch_partial(const float *x, int ldx, int M, const uint16_t *w, int K, in
     launch_partial3(x, ldx, M, w, N, nullptr, 0, nullptr, 0, K, S, part, ldp, p_off, flag, st);
 }
 
-void launch_resid_norm(const float *part, int S, const float *src, float *x, const float *w, float eps, float *xn, int M,
-                       int H, hipStream_t st) {
-    hipLaunchKernelGGL(k_resid_norm, dim3(M), dim3(BT), 0, st, part, S, src, x, w, eps, xn, M, H);
-}
-
-void launch_swiglu(const float *part, int S, int M, int F, float *h, hipStream_t st) {
-    hipLaunchKernelGGL(k_swiglu, dim3(M), dim3(BT), 0, st, part, S, M, F, h);
-}
-
-void launch_finish_linear(const float *part, int S, int M, int N, const float *bias, const float *residual, int act, float *y,
-                          int ldy, hipStream_t st) {
-    hipLaunchKernelGGL(k_finish_linear, dim3(M), dim3(BT), 0, st, part, S, M, N, bias, residual, act, y, ldy);
-}
-
 bool linear_shape_ok(const float *x, int ldx, int M, const uint16_t *w, int K, int N) {
     return M > 0 && K > 0 && N > 0 && K % 32 == 0 && N % 64 == 0 && ldx % 4 == 0 && ldx >= K &&
            (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
@@ -512,8 +463,8 @@ __global__ void __launch_bounds__(HD / 2) k_rotation(const float *invf, float *r
     gst(rot + blockIdx.x * HD + HD / 2 + threadIdx.x, sn);
 }
 
-// xn = RMSNorm(row m of the tiled residual stream x) * w: k_resid_norm's arithmetic for one row
-// (thread i holds elements 4i .. 4i + 3, the same sum order), reading x in the tile layout.
+// xn = RMSNorm(row m of the tiled residual stream x) * w (k_rmsnorm, kernels.h:342-350); thread i holds
+// elements 4i .. 4i + 3.
 __global__ void __launch_bounds__(BT) k_tiled_row_norm(const float *x, int m, const float *w, float eps, float *xn, int H,
                                                        float *xn2) {
     __shared__ float red[4];
