@@ -268,8 +268,10 @@ __global__ void __launch_bounds__(BT) k_conv_mfma(ConvArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 bad |= !(fabsf(v[e]) < 65504.f);
-                h[e] = static_cast<_Float16>(v[e]);
-                o[e] = static_cast<_Float16>(v[e] - static_cast<float>(h[e]));
+                _Float16 he, oe;
+                f16_pair(v[e], he, oe);
+                h[e] = he;
+                o[e] = oe;
             }
             *reinterpret_cast<half4v *>(&whi[r][c4]) = h;
             *reinterpret_cast<half4v *>(&wlo[r][c4]) = o;
@@ -818,9 +820,10 @@ __global__ void __launch_bounds__(BT) k_unit(UnitArgs u) {
             for (int r = 0; r < 16; ++r) {
                 const int row = wr + 8 * (r / 4) + 4 * (l >> 5) + (r & 3), co = wc + 32 * c + (l & 31);
                 if (t0 + row < u.T) bad |= !(fabsf(z[r]) < 65504.f);
-                const _Float16 h = static_cast<_Float16>(z[r]);
+                _Float16 h, o;
+                f16_pair(z[r], h, o);
                 mhi[row * LDM + co] = h;
-                mlo[row * LDM + co] = static_cast<_Float16>(z[r] - static_cast<float>(h));
+                mlo[row * LDM + co] = o;
             }
         }
     if (bad) gst(u.flag, 1u);

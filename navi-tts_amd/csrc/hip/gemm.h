@@ -75,14 +75,6 @@ typedef _Float16 ghalf4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ bool outside_f16(float v) { return !(fabsf(v) < 65504.f); }
 
-// The f16 pair of an f32 value: of the rounded one, as a reader of the stored value would split it. Without
-// the barrier the compiler folds a product that v is into the conversion and the difference.
-__device__ __forceinline__ void f16_pair(float v, _Float16 &h, _Float16 &o) {
-    asm("" : "+v"(v));
-    h = static_cast<_Float16>(v);
-    o = static_cast<_Float16>(v - static_cast<float>(h));
-}
-
 // One value of an f16-pair row.
 __device__ __forceinline__ void split_store(uint16_t *dst, float v, bool &bad) {
     bad |= outside_f16(v);
@@ -259,9 +251,10 @@ __global__ void __launch_bounds__(NW * WAVE, WPS) k_gemm(GemmArgs a) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 ss[i] = fmaf(v[j], v[j], ss[i]);
-                const float q1 = j < 4 ? l0[j & 3] : l1[j & 3];
-                hi[j] = static_cast<_Float16>(v[j] * q1);
-                lo[j] = static_cast<_Float16>(fmaf(v[j], q1, -static_cast<float>(hi[j])));   // the product's own low part
+                _Float16 h, o;
+                f16_pair(v[j] * (j < 4 ? l0[j & 3] : l1[j & 3]), h, o);
+                hi[j] = h;
+                lo[j] = o;
             }
         } else {
             __builtin_memcpy(&hi, &fx[slot][i][0], 16);

@@ -163,9 +163,10 @@ __global__ void __launch_bounds__(NWV * WAVE) k_rows(RowArgs a) {
                     v *= lv[st][j >> 2][j & 3];
                 }
                 bad |= !(fabsf(v) < 65504.f);
-                const _Float16 h = static_cast<_Float16>(v);
+                _Float16 h, o;
+                f16_pair(v, h, o);
                 hi[j] = h;
-                lo[j] = static_cast<_Float16>(v - static_cast<float>(h));
+                lo[j] = o;
             }
 #pragma unroll
             for (int t = 0; t < NT; ++t)
