@@ -6,6 +6,7 @@
 #pragma once
 
 #include "dev_common.h"
+#include "f16_pair.h"
 #include "snake.h"
 
 namespace navi_amd {

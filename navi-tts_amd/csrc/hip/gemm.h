@@ -19,9 +19,9 @@
 // What bounds them: the operand bytes into a CU (about 70 GB/s from L2), then the exchange and the waits of
 // the end. Against the row kernels (16-row blocks, which read every weight once per 16 rows): a prefill of
 // 65 rows 1.22 -> 1.06 ms, 130 1.85 -> 1.34, 300 3.01 -> 1.64, 768 6.66 -> 3.26, 1001 9.24 -> 3.92.
-// Four waves of longer runs, whose sums start from zero at every step, exchange half as much (256 rows 1.44
-// ms instead of 1.66, with the attention on the matrix cores; 768 2.80, 1001 3.32), but give other bits: K/V rows are then up to
-// 12 % further from 64 bits in the layers between the first and the last, and a row's results depend on
+// Four waves of longer runs, whose sums start from zero at every step, exchange half as much and take the
+// norm's sums from the previous launch (256 rows 1.44 ms, with the attention on the matrix cores; 768 2.80, 1001 3.32).
+// They are no further from 64 bits, but have other bits than the row kernels: a row's results then depend on
 // the length of its prompt.
 #pragma once
 

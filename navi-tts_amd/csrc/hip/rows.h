@@ -5,6 +5,7 @@
 #pragma once
 
 #include "dev_common.h"
+#include "f16_pair.h"
 
 namespace navi_amd {
 namespace rows {
